@@ -51,9 +51,11 @@ struct Staging {
     bool pending = false;
   };
   std::vector<Buf> bufs;
-  int get(size_t bytes, void** out) {
+  // `keep`: a buffer still being read by the caller, not handed out.
+  int get(size_t bytes, void** out, int keep = -1) {
     for (size_t i = 0; i < bufs.size(); ++i) {
       Buf& b = bufs[i];
+      if ((int)i == keep) continue;
       if (b.pending) {
         if (hipEventQuery(b.ev) == hipSuccess) b.pending = false;
         else continue;
@@ -934,6 +936,42 @@ void reap_marks(oidt_batch* b) {
   }
 }
 
+// Bytes of one read-back piece: pieces alternate between two pinned buffers,
+// so the host copies one to the caller while the GPU fills the other.
+constexpr size_t kReadPiece = (size_t)4 << 20;
+
+// Packs `rows` rows of `row_len` values (`pitch` values apart on the device)
+// into the caller's contiguous array.  The batch stream must be idle or hold
+// only work that may precede the read.
+template <typename U>
+int read_rows(oidt_batch* b, const char* src, size_t pitch, size_t row_len, size_t rows, void* host) {
+  const size_t per = std::max<size_t>(1, std::min(rows, kReadPiece / (row_len * sizeof(U))));
+  struct Piece { int id; void* p; size_t row0, n; };
+  Piece prev{-1, nullptr, 0, 0};
+  auto drain = [&](const Piece& pc) -> int {
+    HIP_TRY(hipEventSynchronize(b->staging.bufs[pc.id].ev));
+    std::memcpy(static_cast<U*>(host) + pc.row0 * row_len, pc.p, pc.n * row_len * sizeof(U));
+    b->staging.bufs[pc.id].pending = false;
+    return OIDT_OK;
+  };
+  int rc = OIDT_OK;
+  for (size_t r = 0; r < rows && rc == OIDT_OK; r += per) {
+    Piece pc{-1, nullptr, r, std::min(per, rows - r)};
+    // a piece not yet copied out is pending, so the pool hands out another buffer
+    pc.id = b->staging.get(pc.n * row_len * sizeof(U), &pc.p, prev.id);
+    if (pc.id < 0) return fail(OIDT_ENOMEM, "pinned staging allocation failed");
+    const size_t n = pc.n * row_len;
+    hipLaunchKernelGGL((k_pack_rows<U>), dim3((unsigned)std::min<size_t>((n + kThreads - 1) / kThreads, 2048)),
+                       dim3(kThreads), 0, b->stream, reinterpret_cast<const U*>(src), (unsigned)pitch,
+                       (unsigned)row_len, (unsigned)pc.row0, (unsigned)pc.n, static_cast<U*>(pc.p));
+    HIP_TRY(hipGetLastError());
+    if (b->staging.submit(pc.id, b->stream) != 0) return fail(OIDT_EHIP, "event record failed");
+    if (prev.id >= 0) rc = drain(prev);
+    prev = pc;
+  }
+  return rc == OIDT_OK && prev.id >= 0 ? drain(prev) : rc;
+}
+
 // True once the GPU has completed every chunk the run needs (later chunks skip it).
 bool slot_finished(oidt_batch* b, const SlotHost& sh) {
   reap_marks(b);
@@ -1329,8 +1367,9 @@ int oidt_batch_read_field(oidt_batch* b, int32_t slot, int32_t field, void* host
   const size_t prow = (is3d ? (size_t)(d.precision == OIDT_F64 ? padded<double>(d).nz : padded<float>(d).nz)
                             : (size_t)(d.precision == OIDT_F64 ? padded<double>(d).ny : padded<float>(d).ny)) * es;
   const size_t rows = bytes / row;
-  HIP_TRY(hipMemcpy2D(host, row, static_cast<char*>(sh.dmem) + off, prow, row, rows, hipMemcpyDeviceToHost));
-  return OIDT_OK;
+  const char* src = static_cast<const char*>(sh.dmem) + off;
+  return es == 8 ? read_rows<unsigned long long>(b, src, prow / es, row / es, rows, host)
+                 : read_rows<unsigned>(b, src, prow / es, row / es, rows, host);
 }
 
 int oidt_batch_remove(oidt_batch* b, int32_t slot) {
