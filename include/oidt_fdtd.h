@@ -288,7 +288,11 @@ int oidt_batch_remove(oidt_batch* b, int32_t slot);
  * blocked step, TMz, TEz and 3D, xchunk = steps per launch, 2, 4 or 8 in 2D,
  * 2 in 3D).  Once a run
  * has started, its form cannot change between two-kernel, fused and blocked,
- * nor the blocked step's depth (OIDT_ESTATE).
+ * nor the blocked step's depth (OIDT_ESTATE).  Until the first call the library
+ * picks the form itself: TMz and TEz batches without field monitors step in
+ * the blocked form, 8 steps per launch (FP32: the two-kernel form's bits), and
+ * oidt_batch_get_launch returns the defaults above, which a call with zeros
+ * keeps.
  * No counterpart in the reference (fixed launch shapes, fdtd_main.py:263-273). */
 int oidt_batch_set_launch(oidt_batch* b, int32_t xchunk, int32_t grid_blocks, int32_t variant);
 

@@ -9,7 +9,7 @@ import sys
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
 SRC = [os.path.join(HERE, 'csrc', 'fdtd_api.hip')]
-DEPS = [os.path.join(HERE, 'csrc', f) for f in ('fdtd_kernels.h', 'fdtd_slot.h')] + \
+DEPS = [os.path.join(HERE, 'csrc', f) for f in ('fdtd_kernels.h', 'fdtd_blocked2d.h', 'fdtd_slot.h')] + \
        [os.path.join(ROOT, 'include', 'oidt_fdtd.h')]
 LIB = os.path.join(HERE, 'liboidt_fdtd.so')
 ARCH = os.environ.get('OIDT_OFFLOAD_ARCH', 'gfx950')

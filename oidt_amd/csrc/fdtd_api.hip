@@ -20,6 +20,7 @@
 
 #include "../../include/oidt_fdtd.h"
 #include "fdtd_kernels.h"
+#include "fdtd_blocked2d.h"
 
 using namespace oidt;
 
@@ -106,6 +107,10 @@ struct SlotHost {
   // temporally blocked step.  After `steps` completed steps the state is in
   // set B when ceil(steps / tb) is odd.
   int tb = 0;
+  // The same for the form that steps the run's latest chunk, which differs
+  // where the library picks the form (see resolve_form): set at each rebuild
+  // while the run has chunks left.
+  int tb_run = 0;
   int nplanes = 0, nq = 0, wcells = 0, pcells = 0, wyn = 0;
   std::vector<MonHost> mons;
 };
@@ -311,6 +316,12 @@ struct oidt_batch {
   // resident runs' fields exceed the last-level cache (see rebuild_lists)
   bool stream_loads = false;
   int variant = 2;
+  // oidt_batch_set_launch has not been called: the library picks the form
+  // (resolve_form).
+  bool auto_form = true;
+  // The form and depth the launches use: variant / xchunk unless auto_form.
+  int run_variant = 2, run_xchunk = 4;
+  int tb_planes = 32;   // blocked 2D step: planes of its extended tile
   int64_t chunks_enqueued = 0;
   int64_t chunks_done = 0;
   std::deque<std::pair<hipEvent_t, int64_t>> marks;
@@ -520,7 +531,7 @@ int run_tb(int variant, int xchunk) { return variant == 4 ? xchunk : (variant ==
 
 // Kernels whose tiles are per wavefront (four tiles per block): the fused
 // 2D steps.
-bool march_tiles(const oidt_batch* b) { return b->variant == 3; }
+bool march_tiles(const oidt_batch* b) { return b->run_variant == 3; }
 
 // z-cells a wave of the fused 3D step owns (its lane 0 is the cell below).
 constexpr int kHaloZ = kBX - 1;
@@ -528,6 +539,34 @@ constexpr int kHaloZ = kBX - 1;
 // Waves (rows) of a blocked 3D step's block: 16 in FP32; 8 in FP64, whose
 // cells take twice the registers.
 int tb3_waves(int precision) { return precision == OIDT_F64 ? 8 : 16; }
+
+// The form the launches use.  Where the caller has not set the launch knobs
+// (to keep them counts too), TMz and TEz runs without field monitors take the blocked step at its largest depth: a field passes
+// through HBM once per 8 steps and the launches fall from 64 to 4 per chunk.
+// Two-kernel / blocked, us per step: 140 x 72 10.5 / 1.6, 600 x 240 FP64 11.1 /
+// 2.0, 1480 x 430 12.6 / 2.5, 64 guides of 800..4000 x 240 353 / 57.  It gives
+// the two-kernel form's bits, and at a chunk boundary every run's state is
+// back in field set A, so a batch may change between the two there (a
+// monitored run joins or leaves).
+void resolve_form(oidt_batch* b) {
+  b->run_variant = b->variant;
+  b->run_xchunk = b->xchunk;
+  if (b->auto_form && (b->scheme == SCHEME_TMZ || b->scheme == SCHEME_TEZ) && !b->has_monitors()) {
+    b->run_variant = 4;
+    b->run_xchunk = 8;
+  }
+  // Its lanes address the high-side y psi from the low-side array by a 32-bit
+  // offset (three slabs in between): runs beyond that take the two-kernel form.
+  if (b->run_variant == 4 && b->scheme != SCHEME_3D)
+    for (const auto& sh : b->slots)
+      if (sh.used && 3.0 * ((double)sh.desc.nx * sh.desc.num_cpml * (b->precision == OIDT_F64 ? 8 : 4) + 256.0) > 4294967295.0) {
+        b->run_variant = 2;
+        b->run_xchunk = 4;
+      }
+  for (auto& sh : b->slots)
+    if (sh.used && (b->chunks_enqueued - sh.admit_chunk) * kChunk < sh.desc.nt)
+      sh.tb_run = run_tb(b->run_variant, b->run_xchunk);
+}
 
 // Monitor table and the two work lists (after the E and after the H
 // half-step): one item per kMonCells consecutive box cells.
@@ -576,44 +615,46 @@ int rebuild_monitors(oidt_batch* b) {
   return OIDT_OK;
 }
 
+// Extended planes of a blocked 2D step's tiles.  Narrow while every narrow
+// tile gets a CU of its own (see launch_blocked2d): the launch is then one
+// tile's time, and the narrow one is shorter.
+constexpr int kTbNarrow = 32, kTbWide = 48;
+int blocked2d_planes(const oidt_batch* b) {
+  if (b->run_xchunk != 8) return kTbNarrow;
+  size_t tiles = 0;
+  const int tx = kTbNarrow - 2 * 8, ty = 64 - 2 * 8;
+  for (const auto& sh : b->slots)
+    if (sh.used) tiles += (size_t)((sh.desc.nx + tx - 1) / tx) * ((sh.desc.ny + ty - 1) / ty);
+  return tiles <= 256 ? kTbNarrow : kTbWide;
+}
+
 // Rebuild the tile and DFT work lists for the resident slots and upload them.
 int rebuild_lists(oidt_batch* b) {
+  resolve_form(b);
+  if (b->run_variant == 4 && b->scheme != SCHEME_3D) b->tb_planes = blocked2d_planes(b);
   std::vector<int4> tiles, work;
-  const int xc = b->xchunk;
+  const int xc = b->run_xchunk;
   for (int si = 0; si < (int)b->slots.size(); ++si) {
     const SlotHost& sh = b->slots[si];
     if (!sh.used) continue;
     const oidt_run_desc& d = sh.desc;
-    if (d.scheme == SCHEME_3D && b->variant == 3) {
+    if (d.scheme == SCHEME_3D && b->run_variant == 3) {
       // fused step: one wavefront per (row, 63 z-cells) x xc planes
       for (int x0 = 0; x0 < d.nx; x0 += xc)
         for (int y0 = 0; y0 < d.ny; ++y0)
           for (int z0 = 0; z0 < d.nz; z0 += kHaloZ) tiles.push_back(make_int4(si, x0, y0, z0));
-    } else if (d.scheme == SCHEME_3D && b->variant == 4) {
+    } else if (d.scheme == SCHEME_3D && b->run_variant == 4) {
       // blocked 3D step: one block per segment of kTb3Seg planes by its inner
       // rows and z-cells
       const int ty = tb3_waves(b->precision) - 2 * xc, tz = kBX - 2 * xc;
       for (int x0 = 0; x0 < d.nx; x0 += kTb3Seg)
         for (int y0 = 0; y0 < d.ny; y0 += ty)
           for (int z0 = 0; z0 < d.nz; z0 += tz) tiles.push_back(make_int4(si, x0, y0, z0));
-    } else if (b->variant == 4) {
-      // blocked step: one block per tile of its inner cells.  w = 1 marks an
-      // interior tile: its extended tile lies inside every update range and
-      // outside the CPML slabs and the source box, and no capture plane
-      // falls among its inner planes
-      const int tx = kTbPlanes - 2 * xc, ty = 64 - 2 * xc;
-      const int xlo = d.offset + d.num_cpml, xhi = d.nx - d.offset - d.num_cpml;
-      const int ylo = d.offset + d.num_cpml, yhi = d.ny - d.offset - d.num_cpml;
+    } else if (b->run_variant == 4) {
+      // blocked 2D step: one block per tile of its inner cells
+      const int tx = b->tb_planes - 2 * xc, ty = 64 - 2 * xc;
       for (int x0 = 0; x0 < d.nx; x0 += tx)
-        for (int y0 = 0; y0 < d.ny; y0 += ty) {
-          const int ex0 = x0 - xc, ex1 = ex0 + kTbPlanes, ey0 = y0 - xc, ey1 = ey0 + 64;
-          bool in = ex0 >= xlo && ex1 <= xhi && ey0 >= ylo && ey1 <= yhi;
-          if (d.src_field >= 0 && ex0 < d.src_box[1] && ex1 > d.src_box[0] && ey0 < d.src_box[3] && ey1 > d.src_box[2])
-            in = false;
-          for (const int pl : {d.port[0], d.port[0] + 1, d.port[1], d.port[1] + 1})
-            if (pl >= x0 && pl < x0 + tx) in = false;
-          tiles.push_back(make_int4(si, x0, y0, in ? 1 : 0));
-        }
+        for (int y0 = 0; y0 < d.ny; y0 += ty) tiles.push_back(make_int4(si, x0, y0, 0));
     } else if (d.scheme == SCHEME_3D) {
       for (int x0 = 0; x0 < d.nx; x0 += xc)
         for (int y0 = 0; y0 < d.ny; y0 += kBY)
@@ -677,7 +718,7 @@ void launch_half(oidt_batch* b, int gs, int tstep, bool e_half) {
   const Slot<T>* sl = static_cast<const Slot<T>*>(b->d_slots);
   const dim3 blk(kBX, kBY), grd(gs);
   hipStream_t st = b->stream;
-  const bool v1 = b->variant == 1;
+  const bool v1 = b->run_variant == 1;
   switch (b->scheme) {
     case SCHEME_TMZ:
       if (e_half) {
@@ -730,25 +771,47 @@ void launch_fused(oidt_batch* b, int gs, int tstep) {
   }
 }
 
-// The temporally blocked 2D step (TMz, TEz): xchunk steps per launch.  Blocks of 16
-// waves x 2 planes in FP64 (half the registers per wave of 8 x 4, and the
-// FP64 workloads are single small runs that need the extra waves per tile to
-// hide latency), 8 x 4 in FP32 (better on large batches).  The shape depends
-// only on the precision, so a run gives the same bits alone and in a batch.
-template <typename T, int TB, int W>
-void launch_blocked_w(oidt_batch* b, int gs, int tstep) {
+// The temporally blocked 2D step (TMz, TEz), TB steps per launch.  Shapes, as
+// waves x planes per wave (the bits do not depend on them):
+//   narrow, 16 x 2 planes: the shortest step, for grids of few tiles;
+//   wide, 48 planes, 2 x instead of 2.7 x the owned cells stepped: 12 x 4 with
+//     two blocks per CU (TMz FP32), 8 x 6 (TEz FP32, whose second coefficient
+//     would spill in 12 x 4) and 12 x 4 with one block (FP64).
+// us per step, narrow / wide: 600 x 240 1.65 / 1.98 (TMz FP32), 2.05 / 2.29
+// (TMz FP64); 1237 x 301 2.72 / 2.01 and 3.32 / 2.83; 64 guides of 800..4000 x
+// 240 155 / 57 (TMz FP32) and 158 / 59 (TEz FP32; 12 x 4: 69).  8 x 4 (the
+// depths 2 and 4 in FP32) takes 65 and 82 there, 8 x 8 tiles of 64 planes 67.
+template <typename T, int SCH, int TB>
+void launch_blocked2d(oidt_batch* b, int gs, int tstep) {
   const Slot<T>* sl = static_cast<const Slot<T>*>(b->d_slots);
-  if (b->scheme == SCHEME_TEZ)
-    hipLaunchKernelGGL((k_tez_tb<T, TB, W>), dim3(gs), dim3(64, W), 0, b->stream, sl, b->d_tiles, b->d_counts, tstep);
-  else
-    hipLaunchKernelGGL((k_tmz_tb<T, TB, W>), dim3(gs), dim3(64, W), 0, b->stream, sl, b->d_tiles, b->d_counts, tstep);
+  auto go = [&](auto w, auto k, auto mw) {
+    constexpr int W = decltype(w)::value, K = decltype(k)::value, MW = decltype(mw)::value;
+    if constexpr (SCH == SCHEME_TMZ)
+      hipLaunchKernelGGL((k_tmz_tb<T, TB, W, K, MW>), dim3(gs), dim3(64, W), 0, b->stream, sl, b->d_tiles, b->ntiles, tstep);
+    else
+      hipLaunchKernelGGL((k_tez_tb<T, TB, W, K, MW>), dim3(gs), dim3(64, W), 0, b->stream, sl, b->d_tiles, b->ntiles, tstep);
+  };
+  using std::integral_constant;
+  using i2 = integral_constant<int, 2>; using i3 = integral_constant<int, 3>; using i4 = integral_constant<int, 4>;
+  using i6 = integral_constant<int, 6>; using i8 = integral_constant<int, 8>; using i12 = integral_constant<int, 12>;
+  using i16 = integral_constant<int, 16>;
+  if constexpr (TB == 8) {
+    if (b->tb_planes == kTbWide) {
+      if constexpr (sizeof(T) == 8) go(i12{}, i4{}, i3{});
+      else if constexpr (SCH == SCHEME_TEZ) go(i8{}, i6{}, i4{});
+      else go(i12{}, i4{}, i6{});
+      return;
+    }
+  }
+  if constexpr (sizeof(T) == 8 || TB == 8) go(i16{}, i2{}, i4{});
+  else go(i8{}, i4{}, i4{});
 }
-template <typename T, int W>
-void launch_blocked_tb(oidt_batch* b, int gs, int tstep) {
-  switch (b->xchunk) {
-    case 2: launch_blocked_w<T, 2, W>(b, gs, tstep); break;
-    case 4: launch_blocked_w<T, 4, W>(b, gs, tstep); break;
-    default: launch_blocked_w<T, 8, W>(b, gs, tstep); break;
+template <typename T, int SCH>
+void launch_blocked2d_tb(oidt_batch* b, int gs, int tstep) {
+  switch (b->run_xchunk) {
+    case 2: launch_blocked2d<T, SCH, 2>(b, gs, tstep); break;
+    case 4: launch_blocked2d<T, SCH, 4>(b, gs, tstep); break;
+    default: launch_blocked2d<T, SCH, 8>(b, gs, tstep); break;
   }
 }
 // The temporally blocked 3D step: 2 steps per launch, blocks of
@@ -763,22 +826,22 @@ void launch_blocked3d(oidt_batch* b, int gs, int tstep) {
 template <typename T>
 void launch_blocked(oidt_batch* b, int gs, int tstep) {
   if (b->scheme == SCHEME_3D) launch_blocked3d<T>(b, gs, tstep);
-  else if (sizeof(T) == 8) launch_blocked_tb<T, 16>(b, gs, tstep);
-  else launch_blocked_tb<T, 8>(b, gs, tstep);
+  else if (b->scheme == SCHEME_TEZ) launch_blocked2d_tb<T, SCHEME_TEZ>(b, gs, tstep);
+  else launch_blocked2d_tb<T, SCHEME_TMZ>(b, gs, tstep);
 }
 
 // Steps one stencil launch advances: the blocked step's depth, else 1.
-int launch_steps(const oidt_batch* b) { return b->variant == 4 ? b->xchunk : 1; }
+int launch_steps(const oidt_batch* b) { return b->run_variant == 4 ? b->run_xchunk : 1; }
 
 template <typename T>
 void launch_stencil(oidt_batch* b, int gs, int tstep, bool e_half) {
-  if (b->variant == 4) {
+  if (b->run_variant == 4) {
     if (e_half) launch_blocked<T>(b, gs, tstep);
     return;
   }
-  if (b->variant == 3) {
+  if (b->run_variant == 3) {
     if (!e_half) return;
-    switch (b->xchunk) {
+    switch (b->run_xchunk) {
       case 1: launch_fused<T, 1>(b, gs, tstep); break;
       case 2: launch_fused<T, 2>(b, gs, tstep); break;
       case 4: launch_fused<T, 4>(b, gs, tstep); break;
@@ -791,7 +854,7 @@ void launch_stencil(oidt_batch* b, int gs, int tstep, bool e_half) {
     }
     return;
   }
-  switch (b->xchunk) {
+  switch (b->run_xchunk) {
     case 1: launch_half<T, 1>(b, gs, tstep, e_half); break;
     case 2: launch_half<T, 2>(b, gs, tstep, e_half); break;
     case 4: launch_half<T, 4>(b, gs, tstep, e_half); break;
@@ -813,14 +876,15 @@ void launch_advance(oidt_batch* b) {
                      static_cast<Slot<T>*>(b->d_slots), b->max_slots);
 }
 
-// Grid of the stencil launches.  The marching step gives every wave exactly
-// one tile (no cap): a wave holding a second tile at the end of the launch
+// Grid of the stencil launches.  The marching step and the blocked 2D step give
+// every wave / block exactly one tile (no cap): a wave holding a second tile at the end of the launch
 // leaves a tail that measured 15-30 % of the step.  The other forms keep a
 // persistent grid of at most 8192 blocks unless overridden.
 int stencil_grid(const oidt_batch* b) {
   const bool m = march_tiles(b);
   const int items = m ? (b->ntiles + kBY - 1) / kBY : b->ntiles;
-  return grid_for(items, b->grid_override > 0 ? b->grid_override : (m ? (1 << 24) : 8192));
+  const bool once = m || (b->run_variant == 4 && b->scheme != SCHEME_3D);
+  return grid_for(items, b->grid_override > 0 ? b->grid_override : (once ? (1 << 24) : 8192));
 }
 int dft_grid(const oidt_batch* b) { return grid_for(b->nwork, 8192); }
 
@@ -838,7 +902,7 @@ int enqueue_chunk(oidt_batch* b) {
   for (int t = 0; t < kChunk; t += launch_steps(b)) {
     launch_stencil<T>(b, gs, t, true);
     launch_monitors<T>(b, t, 0);
-    if (b->variant < 3) launch_stencil<T>(b, gs, t, false);
+    if (b->run_variant < 3) launch_stencil<T>(b, gs, t, false);
     launch_monitors<T>(b, t, 1);
   }
   launch_dft<T>(b, gd);
@@ -870,7 +934,7 @@ int profile_chunks(oidt_batch* b, int nchunks, double* out) {
   int rc;
   const int per = launch_steps(b);
   for (int c = 0; c < nchunks; ++c) {
-    if (b->variant >= 3) {
+    if (b->run_variant >= 3) {
       if ((rc = timed(0, kChunk / per, [&] {
              for (int t = 0; t < kChunk; t += per) launch_stencil<T>(b, gs, t, true);
            })) != OIDT_OK)
@@ -1067,7 +1131,8 @@ int oidt_batch_create(int32_t scheme, int32_t precision, int32_t max_slots, oidt
   }
 
   // measured defaults on MI355X: the prefetching march over 4-plane tiles in
-  // 3D, the batched-load form with four cells per thread in 2D
+  // 3D, the batched-load form with four cells per thread in 2D (where
+  // resolve_form does not take the blocked step instead)
   b->variant = scheme == SCHEME_3D ? 1 : 2;
   b->xchunk = 4;
   b->slots.resize(max_slots);
@@ -1144,6 +1209,7 @@ int oidt_batch_set_launch(oidt_batch* b, int32_t xchunk, int32_t grid_blocks, in
   if (variant >= 3 && b->has_monitors())
     return fail(OIDT_ESTATE, "field monitors need a two-kernel form (variant 1 or 2)");
   b->variant = variant;
+  b->auto_form = false;
   for (auto& sh : b->slots)
     if (sh.used && b->chunks_enqueued == sh.admit_chunk) sh.tb = run_tb(variant, xc);
   if (xchunk) b->xchunk = xchunk;
@@ -1357,9 +1423,9 @@ int oidt_batch_read_field(oidt_batch* b, int32_t slot, int32_t field, void* host
   if (!host || nbytes != bytes) return fail(OIDT_EINVAL, "host buffer size mismatch");
   HIP_TRY(hipStreamSynchronize(b->stream));
   reap_marks(b);
-  // The fused and blocked steps alternate field sets (see SlotHost::tb).
+  // The fused and blocked steps alternate field sets (see SlotHost::tb_run).
   const int64_t steps = std::min<int64_t>(d.nt, std::max<int64_t>(0, b->chunks_done - sh.admit_chunk) * kChunk);
-  const bool in_b = sh.tb > 0 && (((steps + sh.tb - 1) / sh.tb) & 1);
+  const bool in_b = sh.tb_run > 0 && (((steps + sh.tb_run - 1) / sh.tb_run) & 1);
   const size_t off = d.precision == OIDT_F64 ? (in_b ? layout<double>(d).off_f2[field] : layout<double>(d).off_f[field])
                                              : (in_b ? layout<float>(d).off_f2[field] : layout<float>(d).off_f[field]);
   const bool is3d = d.scheme == SCHEME_3D;
