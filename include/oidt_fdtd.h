@@ -289,8 +289,10 @@ int oidt_batch_remove(oidt_batch* b, int32_t slot);
  * 2 in 3D).  Once a run
  * has started, its form cannot change between two-kernel, fused and blocked,
  * nor the blocked step's depth (OIDT_ESTATE).  Until the first call the library
- * picks the form itself: TMz and TEz batches without field monitors step in
- * the blocked form, 8 steps per launch (FP32: the two-kernel form's bits), and
+ * picks the form itself: 2D batches whose monitors are single-point running
+ * DFTs it can fold (lossy TMz: one per field, TEz: of Ey and Hz, TMz: none)
+ * step in the blocked form, 8 steps per launch (FP32: the two-kernel form's
+ * bits), and
  * oidt_batch_get_launch returns the defaults above, which a call with zeros
  * keeps.
  * No counterpart in the reference (fixed launch shapes, fdtd_main.py:263-273). */

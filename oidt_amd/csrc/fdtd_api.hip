@@ -334,6 +334,9 @@ struct oidt_batch {
   int4* d_mwork[2] = {nullptr, nullptr};   // monitor work after the E / H half-step
   size_t mwork_cap[2] = {0, 0};
   int nmwork[2] = {0, 0};
+  int2* d_smon = nullptr;      // per slot: first monitor in the table, number of monitors
+  bool tb_mon = false;         // the blocked 2D step folds the monitors
+  bool tb_few = false;         // every narrow tile of the blocked 2D step has a CU of its own
   bool has_monitors() const {
     for (const auto& sh : slots)
       if (sh.used && !sh.mons.empty()) return true;
@@ -540,8 +543,26 @@ constexpr int kHaloZ = kBX - 1;
 // cells take twice the registers.
 int tb3_waves(int precision) { return precision == OIDT_F64 ? 8 : 16; }
 
+// Whether the blocked 2D step can fold the batch's monitors: single-point
+// running DFTs, at most one per field of a run (TEz: of Ey and Hz), as the
+// scattering-loss drivers attach them.
+bool blocked2d_monitors(const oidt_batch* b) {
+  for (const auto& sh : b->slots) {
+    if (!sh.used) continue;
+    unsigned seen = 0;
+    for (const MonHost& mh : sh.mons) {
+      const oidt_monitor_desc& d = mh.d;
+      const unsigned bit = 1u << d.field;
+      if (d.mode != OIDT_MON_DFT || d.npts != 1 || d.off[0][0] || d.off[0][1] || d.off[0][2] || (seen & bit)) return false;
+      if (b->scheme == SCHEME_TMZ || (b->scheme == SCHEME_TEZ && d.field == F_EX)) return false;
+      seen |= bit;
+    }
+  }
+  return true;
+}
+
 // The form the launches use.  Where the caller has not set the launch knobs
-// (to keep them counts too), TMz and TEz runs without field monitors take the blocked step at its largest depth: a field passes
+// (to keep them counts too), 2D runs whose field monitors it can fold take the blocked step at its largest depth: a field passes
 // through HBM once per 8 steps and the launches fall from 64 to 4 per chunk.
 // Two-kernel / blocked, us per step: 140 x 72 10.5 / 1.6, 600 x 240 FP64 11.1 /
 // 2.0, 1480 x 430 12.6 / 2.5, 64 guides of 800..4000 x 240 353 / 57.  It gives
@@ -551,7 +572,7 @@ int tb3_waves(int precision) { return precision == OIDT_F64 ? 8 : 16; }
 void resolve_form(oidt_batch* b) {
   b->run_variant = b->variant;
   b->run_xchunk = b->xchunk;
-  if (b->auto_form && (b->scheme == SCHEME_TMZ || b->scheme == SCHEME_TEZ) && !b->has_monitors()) {
+  if (b->auto_form && b->scheme != SCHEME_3D && blocked2d_monitors(b)) {
     b->run_variant = 4;
     b->run_xchunk = 8;
   }
@@ -574,9 +595,11 @@ template <typename T>
 int rebuild_monitors(oidt_batch* b) {
   std::vector<Monitor<T>> table;
   std::vector<int4> work[2];
+  std::vector<int2> first(b->max_slots, make_int2(0, 0));
   for (int si = 0; si < (int)b->slots.size(); ++si) {
     const SlotHost& sh = b->slots[si];
     if (!sh.used) continue;
+    first[si] = make_int2((int)table.size(), (int)sh.mons.size());
     for (const MonHost& mh : sh.mons) {
       const oidt_monitor_desc& d = mh.d;
       Monitor<T> m{};
@@ -590,6 +613,7 @@ int rebuild_monitors(oidt_batch* b) {
       m.ex = d.box[1] - d.box[0]; m.ey = d.box[3] - d.box[2]; m.ez = d.box[5] - d.box[4];
       m.gx = sh.desc.nx; m.gy = sh.desc.ny; m.gz = sh.desc.nz;
       m.shift = d.shift; m.nrec = d.nrec;
+      m.after_h = d.after_h;
       const int id = (int)table.size();
       table.push_back(m);
       for (size_t c0 = 0; c0 < mh.cells; c0 += kMonCells) work[d.after_h ? 1 : 0].push_back(make_int4(id, (int)c0, 0, 0));
@@ -606,6 +630,9 @@ int rebuild_monitors(oidt_batch* b) {
   }
   if (!table.empty() && (rc = upload_bytes(b, b->d_mons, table.data(), table.size() * sizeof(Monitor<T>))) != OIDT_OK)
     return rc;
+  if (!b->d_smon && hipMallocAsync(reinterpret_cast<void**>(&b->d_smon), b->max_slots * sizeof(int2), b->stream) != hipSuccess)
+    return fail(OIDT_ENOMEM, "monitor index allocation failed");
+  if (!table.empty() && (rc = upload_bytes(b, b->d_smon, first.data(), first.size() * sizeof(int2))) != OIDT_OK) return rc;
   for (int h = 0; h < 2; ++h) {
     if ((rc = grow(b, &b->d_mwork[h], &b->mwork_cap[h], std::max<size_t>(work[h].size(), 1))) != OIDT_OK) return rc;
     if (!work[h].empty() && (rc = upload_bytes(b, b->d_mwork[h], work[h].data(), work[h].size() * sizeof(int4))) != OIDT_OK)
@@ -619,18 +646,20 @@ int rebuild_monitors(oidt_batch* b) {
 // tile gets a CU of its own (see launch_blocked2d): the launch is then one
 // tile's time, and the narrow one is shorter.
 constexpr int kTbNarrow = 32, kTbWide = 48;
-int blocked2d_planes(const oidt_batch* b) {
+int blocked2d_planes(oidt_batch* b) {
   if (b->run_xchunk != 8) return kTbNarrow;
   size_t tiles = 0;
   const int tx = kTbNarrow - 2 * 8, ty = 64 - 2 * 8;
   for (const auto& sh : b->slots)
     if (sh.used) tiles += (size_t)((sh.desc.nx + tx - 1) / tx) * ((sh.desc.ny + ty - 1) / ty);
-  return tiles <= 256 ? kTbNarrow : kTbWide;
+  b->tb_few = tiles <= 256;
+  return b->tb_few || b->tb_mon ? kTbNarrow : kTbWide;
 }
 
 // Rebuild the tile and DFT work lists for the resident slots and upload them.
 int rebuild_lists(oidt_batch* b) {
   resolve_form(b);
+  b->tb_mon = b->run_variant == 4 && b->scheme != SCHEME_3D && b->has_monitors();
   if (b->run_variant == 4 && b->scheme != SCHEME_3D) b->tb_planes = blocked2d_planes(b);
   std::vector<int4> tiles, work;
   const int xc = b->run_xchunk;
@@ -784,27 +813,43 @@ void launch_fused(oidt_batch* b, int gs, int tstep) {
 template <typename T, int SCH, int TB>
 void launch_blocked2d(oidt_batch* b, int gs, int tstep) {
   const Slot<T>* sl = static_cast<const Slot<T>*>(b->d_slots);
-  auto go = [&](auto w, auto k, auto mw) {
-    constexpr int W = decltype(w)::value, K = decltype(k)::value, MW = decltype(mw)::value;
+  const Monitor<T>* mons = static_cast<const Monitor<T>*>(b->d_mons);
+  auto go = [&](auto w, auto k, auto mw, auto mon) {
+    constexpr int W = decltype(w)::value, K = decltype(k)::value, MW = decltype(mw)::value, MON = decltype(mon)::value;
     if constexpr (SCH == SCHEME_TMZ)
       hipLaunchKernelGGL((k_tmz_tb<T, TB, W, K, MW>), dim3(gs), dim3(64, W), 0, b->stream, sl, b->d_tiles, b->ntiles, tstep);
+    else if constexpr (SCH == SCHEME_TEZ)
+      hipLaunchKernelGGL((k_tez_tb<T, TB, W, K, MW, MON>), dim3(gs), dim3(64, W), 0, b->stream, sl, b->d_tiles, b->ntiles,
+                         tstep, mons, b->d_smon);
     else
-      hipLaunchKernelGGL((k_tez_tb<T, TB, W, K, MW>), dim3(gs), dim3(64, W), 0, b->stream, sl, b->d_tiles, b->ntiles, tstep);
+      hipLaunchKernelGGL((k_tmzl_tb<T, TB, W, K, MW, MON>), dim3(gs), dim3(64, W), 0, b->stream, sl, b->d_tiles, b->ntiles,
+                         tstep, mons, b->d_smon);
   };
   using std::integral_constant;
-  using i2 = integral_constant<int, 2>; using i3 = integral_constant<int, 3>; using i4 = integral_constant<int, 4>;
-  using i6 = integral_constant<int, 6>; using i8 = integral_constant<int, 8>; using i12 = integral_constant<int, 12>;
-  using i16 = integral_constant<int, 16>;
+  using i0 = integral_constant<int, 0>; using i2 = integral_constant<int, 2>; using i3 = integral_constant<int, 3>;
+  using i4 = integral_constant<int, 4>; using i6 = integral_constant<int, 6>; using i8 = integral_constant<int, 8>;
+  using i12 = integral_constant<int, 12>; using i16 = integral_constant<int, 16>;
   if constexpr (TB == 8) {
+    if constexpr (SCH != SCHEME_TMZ) {
+      using all = integral_constant<int, SCH == SCHEME_TEZ ? (MON_A | MON_B) : (MON_A | MON_B | MON_C)>;
+      if (b->tb_mon) {
+        // with monitors: 16 x 2 while every tile has a CU of its own, else 8 x
+        // 4 (4170 x 430 TEz, two planes: 15.7 / 11.5 us per step; 287 x 235
+        // lossy TMz, three: 2.9 / 3.5; 48-plane tiles 12.5 and 4.1)
+        if constexpr (sizeof(T) == 4)
+          if (!b->tb_few) return go(i8{}, i4{}, i4{}, all{});
+        return go(i16{}, i2{}, i4{}, all{});
+      }
+    }
     if (b->tb_planes == kTbWide) {
-      if constexpr (sizeof(T) == 8) go(i12{}, i4{}, i3{});
-      else if constexpr (SCH == SCHEME_TEZ) go(i8{}, i6{}, i4{});
-      else go(i12{}, i4{}, i6{});
+      if constexpr (sizeof(T) == 8) go(i12{}, i4{}, i3{}, i0{});
+      else if constexpr (SCH == SCHEME_TMZ) go(i12{}, i4{}, i6{}, i0{});
+      else go(i8{}, i6{}, i4{}, i0{});
       return;
     }
   }
-  if constexpr (sizeof(T) == 8 || TB == 8) go(i16{}, i2{}, i4{});
-  else go(i8{}, i4{}, i4{});
+  if constexpr (sizeof(T) == 8 || TB == 8) go(i16{}, i2{}, i4{}, i0{});
+  else go(i8{}, i4{}, i4{}, i0{});
 }
 template <typename T, int SCH>
 void launch_blocked2d_tb(oidt_batch* b, int gs, int tstep) {
@@ -827,6 +872,7 @@ template <typename T>
 void launch_blocked(oidt_batch* b, int gs, int tstep) {
   if (b->scheme == SCHEME_3D) launch_blocked3d<T>(b, gs, tstep);
   else if (b->scheme == SCHEME_TEZ) launch_blocked2d_tb<T, SCHEME_TEZ>(b, gs, tstep);
+  else if (b->scheme == SCHEME_TMZ_LOSSY) launch_blocked2d<T, SCHEME_TMZ_LOSSY, 8>(b, gs, tstep);
   else launch_blocked2d_tb<T, SCHEME_TMZ>(b, gs, tstep);
 }
 
@@ -901,8 +947,9 @@ int enqueue_chunk(oidt_batch* b) {
   const int gs = stencil_grid(b), gd = dft_grid(b);
   for (int t = 0; t < kChunk; t += launch_steps(b)) {
     launch_stencil<T>(b, gs, t, true);
+    if (b->run_variant >= 3) continue;   // the whole step(s), monitors included
     launch_monitors<T>(b, t, 0);
-    if (b->run_variant < 3) launch_stencil<T>(b, gs, t, false);
+    launch_stencil<T>(b, gs, t, false);
     launch_monitors<T>(b, t, 1);
   }
   launch_dft<T>(b, gd);
@@ -1610,6 +1657,7 @@ int oidt_batch_destroy(oidt_batch* b) {
         if (p) (void)hipFree(p);
   }
   if (b->d_mons) (void)hipFree(b->d_mons);
+  if (b->d_smon) (void)hipFree(b->d_smon);
   for (int h = 0; h < 2; ++h)
     if (b->d_mwork[h]) (void)hipFree(b->d_mwork[h]);
   if (b->gexec) (void)hipGraphExecDestroy(b->gexec);

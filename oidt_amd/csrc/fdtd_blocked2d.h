@@ -27,8 +27,17 @@
 //   - the per-plane 1/kappa stay in scalar registers over the launch.
 //
 // The arithmetic is written with explicit fused multiply-adds, the ones the
-// two-kernel form k_*_e2 / k_*_h2 compiles to, so every shape and every class
-// gives the same bits.
+// two-kernel forms (k_*_e2 / k_*_h2, k_tmzl_e / k_tmzl_h) compile to, so every
+// shape and every class gives the same bits.
+//
+// Field monitors.  The running DFTs of the study drivers (one per field, over
+// any box) ride along: their sums of the wave's cells sit in registers over
+// the launch, each step folded as k_monitor folds it (product and sum in
+// double, rounded to T), so a whole-plane phasor costs one read and one write
+// of its sums per 8 steps instead of a kernel per step.  us per step, two
+// kernels and the monitor kernel / blocked: TEz study 4170 x 430 with two
+// planes 36.8 / 11.5, lossy TMz 2787 x 430 with three 33.2 / 11.4, bound by the
+// conversions and FP64 operations of the fold.
 #pragma once
 #include "fdtd_kernels.h"
 
@@ -95,6 +104,10 @@ struct Blocked2d<SCHEME_TMZ> {
   static constexpr int PX = F_EZ, PY = F_EZ, QX = F_HY, QY = F_HX;   // psi components
   static constexpr int SRC = F_EZ;
 };
+// The lossy TMz form differences the other way round: E reads A at i-1, H
+// reads B at i+1.
+template <>
+struct Blocked2d<SCHEME_TMZ_LOSSY> : Blocked2d<SCHEME_TMZ> {};
 template <>
 struct Blocked2d<SCHEME_TEZ> {
   static constexpr int A = F_HZ, B = F_EY, C = F_EX;
@@ -102,11 +115,31 @@ struct Blocked2d<SCHEME_TEZ> {
   static constexpr int SRC = F_HZ;
 };
 
-template <typename T, int SCH, int TB, int W, int K>
+// CPML cells of the lossy TMz form (k_tmzl_e, k_tmzl_h): row and coefficient
+// are the distance from the grid edge.
+__device__ __forceinline__ int slab_e_lossy(int x, int e, int N, int& d, int& ci) {
+  if (x < N) { d = ci = x; return 0; }
+  if (e - x < N) { d = ci = e - x; return 1; }
+  return -1;
+}
+__device__ __forceinline__ int slab_h_lossy(int x, int e, int N, int& d, int& ci) {
+  if (x >= 1 && x < N) { d = ci = x; return 0; }
+  if (e - 1 - x >= 1 && e - 1 - x < N) { d = ci = e - 1 - x; return 1; }
+  return -1;
+}
+
+// Roles with a monitor, as bits of a kernel's MON.
+enum : int { MON_A = 1, MON_B = 2, MON_C = 4 };
+
+// MON: the roles a run's monitors may take (0: the kernel ignores monitors);
+// smon[slot]: first monitor of the run in `mons` and their number, at most one
+// per field.
+template <typename T, int SCH, int TB, int W, int K, int MON>
 __device__ __forceinline__ void blocked_step_2d(const Slot<T>* __restrict__ slots, const int4* __restrict__ tiles,
-                                                int ntiles, int tstep) {
+                                                int ntiles, int tstep, const Monitor<T>* __restrict__ mons,
+                                                const int2* __restrict__ smon) {
   using R = Blocked2d<SCH>;
-  constexpr bool tm = SCH == SCHEME_TMZ;
+  constexpr bool tm = SCH != SCHEME_TEZ, lossy = SCH == SCHEME_TMZ_LOSSY;
   constexpr int P = W * K;                           // planes of the extended tile
   constexpr int TX = P - 2 * TB, TY = 64 - 2 * TB;   // inner cells of a tile
   static_assert(TX > 0 && TY > 0 && kChunk % TB == 0, "blocking depth");
@@ -158,10 +191,18 @@ __device__ __forceinline__ void blocked_step_2d(const Slot<T>* __restrict__ slot
       m[q] = ldg<uint8_t>(gm, idx);
     }
     // ---- row (y-only) constants of this lane
-    const bool yin = jok && j >= jb && j < je, yin1 = jok && j > jb && j < je;
+    // update rows: TMz Ez, Hy [jb, je), Hx (jb, je); TEz Ex [jb, je), Ey and Hz
+    // (jb, je); lossy TMz E [1, je), H [0, je)
+    const bool yin = jok && j >= jb && j < je, yin1 = jok && (lossy || j > jb) && j < je;
     int dye = 0, cye = 0, dyh = 0, cyh = 0;
-    const int sye = yin ? slab_e(j, jb, je, N, dye, cye) : -1;
-    const int syh = yin1 ? slab_h(j, jb, je, N, dyh, cyh) : -1;
+    auto se = [&](int x, int b_, int e_, int& d, int& ci) {
+      return lossy ? slab_e_lossy(x, e_, N, d, ci) : slab_e(x, b_, e_, N, d, ci);
+    };
+    auto sh = [&](int x, int b_, int e_, int& d, int& ci) {
+      return lossy ? slab_h_lossy(x, e_, N, d, ci) : slab_h(x, b_, e_, N, d, ci);
+    };
+    const int sye = yin ? se(j, jb, je, dye, cye) : -1;
+    const int syh = yin1 ? sh(j, jb, je, dyh, cyh) : -1;
     const T ikye = yin ? ldg<T>(ike1, j * es) : T(0), ikyh = yin1 ? ldg<T>(ikh1, j * es) : T(0);
     const T bey = sye >= 0 ? s.be[cye] : T(0), cey = sye >= 0 ? s.ceo[cye] : T(0);
     const T bhy = syh >= 0 ? s.bh[cyh] : T(0), chy = syh >= 0 ? s.cho[cyh] : T(0);
@@ -170,13 +211,14 @@ __device__ __forceinline__ void blocked_step_2d(const Slot<T>* __restrict__ slot
     // ---- class of this wave (see above)
     const int sx0 = s.sx0, sx1 = s.sx1, port0 = s.port[0], port1 = s.port[1];
     auto meets = [&](int lo, int hi) { return ib0 < hi && ib0 + K > lo; };
-    const bool special = (has_src && meets(sx0, sx1)) || meets(port0, port0 + 2) || meets(port1, port1 + 2);
+    const bool ports = !lossy && s.nf > 0;   // nothing folds the captures of a run without frequencies
+    const bool special = (has_src && meets(sx0, sx1)) || (ports && (meets(port0, port0 + 2) || meets(port1, port1 + 2)));
     const bool xplain = ib0 >= ib + N && ib0 + K <= ie - N && !special;
     const bool yplain = j0 - TB >= jb + N && j0 - TB + 64 <= je - N;
     // Where plane ib0 + l is updated and its x-slab cells, lane l = 0..K-1 (a
     // vector register serves all the wave's planes; the values of one plane
-    // are read from its lane).  Roles: bit 0 x in [ib, ie), 1 x in (ib, ie),
-    // 2 source, 3 E slab, 4 H slab, 5..8 capture at port0, port1, port0 + 1,
+    // are read from its lane).  Roles: bit 0 x in [ib, ie), 1 x in (ib, ie)
+    // (lossy: [0, ie)), 2 source, 3 E slab, 4 H slab, 5..8 capture at port0, port1, port0 + 1,
     // port1 + 1.  re / rh: row of the E / H psi slab, kHi added on its high
     // side.
     constexpr int kHi = 1 << 24;
@@ -185,11 +227,11 @@ __device__ __forceinline__ void blocked_step_2d(const Slot<T>* __restrict__ slot
       XCell x{};
       const int i = ib00 + l;
       const bool iok = i >= 0 && i < nx;
-      const bool xin = iok && i >= ib && i < ie, xin1 = iok && i > ib && i < ie;
-      const bool inner = iok && i >= i0 && i < i0 + TX;
+      const bool xin = iok && i >= ib && i < ie, xin1 = iok && (lossy || i > ib) && i < ie;
+      const bool inner = ports && iok && i >= i0 && i < i0 + TX;
       int dxe = 0, dxh = 0;
-      const int sxe = xin ? slab_e(i, ib, ie, N, dxe, x.cxe) : -1;
-      const int sxh = xin1 ? slab_h(i, ib, ie, N, dxh, x.cxh) : -1;
+      const int sxe = xin ? se(i, ib, ie, dxe, x.cxe) : -1;
+      const int sxh = xin1 ? sh(i, ib, ie, dxh, x.cxh) : -1;
       x.re = dxe + (sxe == 1 ? kHi : 0);
       x.rh = dxh + (sxh == 1 ? kHi : 0);
       x.f = (xin ? 1 : 0) | (xin1 ? 2 : 0) | (iok && i >= sx0 && i < sx1 ? 4 : 0) | (sxe >= 0 ? 8 : 0) |
@@ -198,29 +240,32 @@ __device__ __forceinline__ void blocked_step_2d(const Slot<T>* __restrict__ slot
       return x;
     };
     auto at = [](int v, int q) { return __builtin_amdgcn_readlane(v, q); };
-    // rows of the x psi (TMz: the E / H rows of Ez, Hy; TEz: those of Ey, Hz)
-    const bool yx = tm ? yin : yin1;
+    // rows of the x psi: E (TMz Ez, TEz Ey) and H (TMz Hy, TEz Hz); first
+    // planes of the y psi: E (TMz Ez, TEz Ex) and H (TMz Hx, TEz Hz)
+    const bool yxe = tm ? yin : yin1, yxh = tm && !lossy ? yin : yin1;
+    const int pye = tm ? ib : ib + 1, pyh = lossy ? 0 : pye;
     // ---- coefficients
     T cb0[K], cb1[K], kx[K], kh[K];
     // lane q loads plane q's 1/kappa; each then sits in a scalar register
     T lkx = T(0), lkh = T(0);
     if (lane < K) {
       const int i = ib0 + lane;
-      const bool xin = i >= ib && i < ie, xin1 = i > ib && i < ie;
+      const bool xin = i >= ib && i < ie, xin1 = (lossy ? i >= 0 : i > ib) && i < ie;
       lkx = xin ? ldg<T>(ike0, i * es) : T(0);
       lkh = xin1 ? ldg<T>(ikh0, i * es) : T(0);
     }
-    constexpr int c0 = tm ? 2 : 0;
+    // cb0: TMz cb (lossy CURL_H), TEz cb of Ex; cb1: TEz cb of Ey, lossy MOD_E
+    constexpr int c0 = tm ? 2 : 0, c1 = lossy ? 0 : 1;
     const T v00 = s.cbv[c0][0], v01 = s.cbv[c0][1], v02 = s.cbv[c0][2], v03 = s.cbv[c0][3];
-    const T v10 = s.cbv[1][0], v11 = s.cbv[1][1], v12 = s.cbv[1][2], v13 = s.cbv[1][3];
+    const T v10 = s.cbv[c1][0], v11 = s.cbv[c1][1], v12 = s.cbv[c1][2], v13 = s.cbv[c1][3];
 #pragma unroll
     for (int q = 0; q < K; ++q) {
       kx[q] = lane_get(lkx, q);
       kh[q] = lane_get(lkh, q);
       cb0[q] = cb_of(v00, v01, v02, v03, m[q], c0);
-      cb1[q] = tm ? T(0) : cb_of(v10, v11, v12, v13, m[q], 1);
+      cb1[q] = tm && !lossy ? T(0) : cb_of(v10, v11, v12, v13, m[q], c1);
     }
-    const T db = s.db;
+    const T db = s.db, dxT = s.dxT, dtmu = s.dtmu;
     // CLS 0: anything; 1: bulk only; 2: no x slab or limit, source or capture;
     // 3: no source or capture.
     auto tile = [&](auto cls) {
@@ -247,9 +292,8 @@ __device__ __forceinline__ void blocked_step_2d(const Slot<T>* __restrict__ slot
 #pragma unroll
         for (int q = 0; q < K; ++q) {
           const int i = ib0 + q;
-          const bool in = i >= ib + (tm ? 0 : 1) && i < ie;   // the y psi's planes
-          if (in && sye >= 0) py[q] = ldg<T>(gpy, (unsigned)(i * N) * es + oe);
-          if (in && syh >= 0) qy[q] = ldg<T>(gqy, (unsigned)(i * N) * es + oh);
+          if (i >= pye && i < ie && sye >= 0) py[q] = ldg<T>(gpy, (unsigned)(i * N) * es + oe);
+          if (i >= pyh && i < ie && syh >= 0) qy[q] = ldg<T>(gqy, (unsigned)(i * N) * es + oh);
         }
       }
       // x-slab coefficients, lane q plane q
@@ -265,23 +309,25 @@ __device__ __forceinline__ void blocked_step_2d(const Slot<T>* __restrict__ slot
 #pragma unroll
         for (int q = 0; q < K; ++q) {
           const int f = at(x.f, q), re = at(x.re, q), rh = at(x.rh, q);
-          if ((f & 8) && yx) px[q] = ldg<T>(psiA[psi_id(R::PX, 0, re >= kHi)], (unsigned)((re & (kHi - 1)) * ny + jc) * es);
-          if ((f & 16) && yx) qx[q] = ldg<T>(psiA[psi_id(R::QX, 0, rh >= kHi)], (unsigned)((rh & (kHi - 1)) * ny + jc) * es);
+          if ((f & 8) && yxe) px[q] = ldg<T>(psiA[psi_id(R::PX, 0, re >= kHi)], (unsigned)((re & (kHi - 1)) * ny + jc) * es);
+          if ((f & 16) && yxh) qx[q] = ldg<T>(psiA[psi_id(R::QX, 0, rh >= kHi)], (unsigned)((rh & (kHi - 1)) * ny + jc) * es);
         }
       }
       // A cell outside a component's update range keeps its value by a zero
       // factor (its coefficient, 1/kappa or db), so the steps need no range
       // selects (only a non-finite neighbour could change it).  dbr: db of the
       // rows of TMz Hy / TEz Hz.
-      T dbr = db;
+      T dbr = db, dtr = dtmu;   // dtr: dt / mu of the lossy form's Hy psi
       if (CLS != 1) {
-        dbr = (tm ? yin : yin1) ? db : T(0);
+        dbr = yxh ? db : T(0);
+        dtr = yxh ? dtr : T(0);
 #pragma unroll
         for (int q = 0; q < K; ++q) {
           const int f = kX ? at(lf, q) : 3;
           const bool x0 = (f & 1) != 0, x1 = (f & 2) != 0;
           cb0[q] = (tm ? x0 : x1) && yin ? cb0[q] : T(0);
           if (!tm) cb1[q] = x0 && yin1 ? cb1[q] : T(0);
+          if (lossy) cb1[q] = x0 && yin ? cb1[q] : T(1);
         }
       }
       // With few planes the flags, masks and slab coefficients stay in scalar
@@ -295,11 +341,26 @@ __device__ __forceinline__ void blocked_step_2d(const Slot<T>* __restrict__ slot
       auto cap = [&](int t, int plane, T v) {
         ring[((size_t)(tstep + t) * nplanes + plane) * pcells + cw] = v;
       };
-      // E half-step of plane q; up: A of plane q + 1
+      // E half-step of plane q; up: A of plane q + 1 (lossy: q - 1)
       auto e_half = [&](int q, T up, int t, T jv) {
         const unsigned f = flags(q);
-        const T dx = up - a[q];
-        if constexpr (tm) {
+        const T dx = lossy ? a[q] - up : up - a[q];
+        if constexpr (lossy) {
+          const T dy = lane_prev(c[q]) - c[q];
+          const T ch = cb0[q];
+          T e = fmadd(cb1[q], bf[q], ch * fmadd(dy, ikye, dx * kx[q]));
+          if (kSp && (f & 4u)) e = jsrc ? e - jv : e;
+          if (CLS != 1) {
+            const T chdx = ch * dxT;
+            if (kX && (f & 8u)) {
+              px[q] = fmadd(coef(lce, q), dx, coef(lbe, q) * px[q]);
+              e = fmadd(chdx, px[q], e);
+            }
+            py[q] = fmadd(cey, dy, bey * py[q]);
+            e = sye >= 0 ? fmadd(chdx, py[q], e) : e;
+          }
+          bf[q] = e;
+        } else if constexpr (tm) {
           const T dy = lane_next(c[q]) - c[q];
           const T cb = cb0[q];
           T e = fmadd(cb, fmadd(dx, kx[q], -(dy * ikye)), bf[q]);
@@ -333,12 +394,25 @@ __device__ __forceinline__ void blocked_step_2d(const Slot<T>* __restrict__ slot
           if (f & 64u) cap(t, 3, bf[q]);
         }
       };
-      // H half-step of plane q; dn: B of plane q - 1
+      // H half-step of plane q; dn: B of plane q - 1 (lossy: q + 1)
       auto h_half = [&](int q, T dn, int t, T jv) {
         const unsigned f = flags(q);
-        const T dx = bf[q] - dn;
+        const T dx = lossy ? dn - bf[q] : bf[q] - dn;
         T h;
-        if constexpr (tm) {
+        if constexpr (lossy) {
+          const T dy = bf[q] - lane_next(bf[q]);
+          T hx = fmadd(db * dy, ikyh, c[q]);
+          h = fmadd((CLS != 1 ? dbr : db) * dx, kh[q], a[q]);
+          if (CLS != 1) {
+            if (kX && (f & 16u)) {
+              qx[q] = fmadd(coef(lch, q), dx, coef(lbh, q) * qx[q]);
+              h = fmadd(dtr, qx[q], h);
+            }
+            qy[q] = fmadd(chy, dy, bhy * qy[q]);
+            hx = syh >= 0 ? fmadd(dtmu, qy[q], hx) : hx;
+          }
+          if (!kX || (f & 2u)) c[q] = hx;
+        } else if constexpr (tm) {
           const T dy = bf[q] - lane_prev(bf[q]);
           T hx = fmadd(db * -dy, ikyh, c[q]);
           if (CLS != 1) {
@@ -374,26 +448,112 @@ __device__ __forceinline__ void blocked_step_2d(const Slot<T>* __restrict__ slot
           if (f & 256u) cap(t, 5, h);
         }
       };
-      xA[w][lane] = a[0];
+      // ---- monitors: running sums of this wave's cells, weights (lane t:
+      // record of step n0 + t), steps with a record
+      constexpr int NM = MON == 0 ? 1 : 3;
+      T mre[NM][K], mim[NM][K];
+      double lcr[NM], lci[NM], msc[NM];
+      unsigned mvalid[NM];
+      const Monitor<T>* mon[NM];
+      bool mafter[NM];
+      if constexpr (MON != 0) {
+        const int2 sm = smon[tl.x];
+#pragma unroll
+        for (int r = 0; r < NM; ++r) {
+          mvalid[r] = 0;
+          mon[r] = nullptr;
+          if (!(MON & (1 << r))) continue;
+          const int field = r == 0 ? R::A : r == 1 ? R::B : R::C;
+          for (int k = 0; k < sm.y; ++k)
+            if (mons[sm.x + k].field == field) mon[r] = mons + sm.x + k;
+          lcr[r] = lci[r] = 0.0;
+          if (mon[r]) {
+            const Monitor<T>& m = *mon[r];
+            const int rec = n0 + lane + m.shift;
+            const bool has = lane < nsteps && rec >= 0 && rec < m.nrec;
+            // a wave whose planes all lie in the ghost frame folds nothing
+            mvalid[r] = ib0 + K > i0 && ib0 < i0 + TX ? (unsigned)__ballot(has) : 0u;
+            lcr[r] = has ? m.cs[2 * rec] : 0.0;
+            lci[r] = has ? m.cs[2 * rec + 1] : 0.0;
+            msc[r] = m.scale;
+            mafter[r] = m.after_h != 0;
+#pragma unroll
+            for (int q = 0; q < K; ++q) {
+              const int i = ib0 + q, cell = (i - m.x0) * m.ey + (j - m.y0);
+              const bool in = i >= i0 && i < i0 + TX && i >= m.x0 && i < m.x0 + m.ex && lane >= TB && lane < TB + TY &&
+                              j >= m.y0 && j < m.y0 + m.ey;
+              mre[r][q] = in ? m.re[cell] : T(0);
+              mim[r][q] = in ? m.im[cell] : T(0);
+            }
+          }
+        }
+      }
+      auto fold = [&](int t, bool after) {
+        if constexpr (MON != 0) {
+#pragma unroll
+          for (int r = 0; r < NM; ++r) {
+            if (!(MON & (1 << r)) || !((mvalid[r] >> t) & 1u) || mafter[r] != after) continue;
+            const double cr = lane_get(lcr[r], t), ci = lane_get(lci[r], t), sc = msc[r];
+#pragma unroll
+            for (int q = 0; q < K; ++q) {
+              const double v = sc * (double)(r == 0 ? a[q] : r == 1 ? bf[q] : c[q]);
+              mre[r][q] = (T)fmadd(v, cr, (double)mre[r][q]);
+              mim[r][q] = (T)fmadd(v, ci, (double)mim[r][q]);
+            }
+          }
+        }
+      };
+      // first and last plane in the order of the E half-step: E takes its
+      // neighbour from the wave that holds the plane after `last`, H from the
+      // one before `first`
+      constexpr int first = lossy ? K - 1 : 0, last = lossy ? 0 : K - 1;
+      const bool wnext = lossy ? w > 0 : w + 1 < W, wprev = lossy ? w + 1 < W : w > 0;
+      const int wn = lossy ? w - 1 : w + 1, wp = lossy ? w + 1 : w - 1;
+      xA[w][lane] = a[first];
       for (int t = 0; t < nsteps; ++t) {
         const T jv = kSp ? lane_get(jvl, t) : T(0);
 #pragma unroll
-        for (int q = 0; q + 1 < K; ++q) e_half(q, a[q + 1], t, jv);
+        for (int u = 0; u + 1 < K; ++u) {
+          const int q = lossy ? K - 1 - u : u;
+          e_half(q, a[lossy ? q - 1 : q + 1], t, jv);
+        }
         lds_barrier();
-        e_half(K - 1, w + 1 < W ? xA[w + 1][lane] : a[K - 1], t, jv);
-        xB[w][lane] = bf[K - 1];
+        e_half(last, wnext ? xA[wn][lane] : a[last], t, jv);
+        xB[w][lane] = bf[last];
+        fold(t, false);
 #pragma unroll
-        for (int q = 1; q < K; ++q) h_half(q, bf[q - 1], t, jv);
+        for (int u = 1; u < K; ++u) {
+          const int q = lossy ? K - 1 - u : u;
+          h_half(q, bf[lossy ? q + 1 : q - 1], t, jv);
+        }
         lds_barrier();
-        h_half(0, w > 0 ? xB[w - 1][lane] : bf[0], t, jv);
-        xA[w][lane] = a[0];
+        h_half(first, wprev ? xB[wp][lane] : bf[first], t, jv);
+        xA[w][lane] = a[first];
+        fold(t, true);
+      }
+      if constexpr (MON != 0) {
+#pragma unroll
+        for (int r = 0; r < NM; ++r) {
+          if (!(MON & (1 << r)) || !mvalid[r]) continue;
+          const Monitor<T>& m = *mon[r];
+#pragma unroll
+          for (int q = 0; q < K; ++q) {
+            const int i = ib0 + q, cell = (i - m.x0) * m.ey + (j - m.y0);
+            if (i >= i0 && i < i0 + TX && i >= m.x0 && i < m.x0 + m.ex && lane >= TB && lane < TB + TY && j >= m.y0 &&
+                j < m.y0 + m.ey) {
+              m.re[cell] = mre[r][q];
+              m.im[cell] = mim[r][q];
+            }
+          }
+        }
       }
       // ---- the inner cells to set B (fields unconditionally: cells no step
       // updates hold the same value in both sets)
       const int ib1 = opaque_uniform(ib00);
       const int js = j0 - TB + opaque_value(lane);
       const bool own = js >= j0 && js < j0 + TY && js < ny;   // j0 >= 0
-      const bool yins = js >= jb && js < je, yins1 = js > jb && js < je, yxs = tm ? yins : yins1;
+      const bool yins = js >= jb && js < je, yins1 = (lossy || js > jb) && js < je;
+      const bool yxes = tm ? yins : yins1, yxhs = tm && !lossy ? yins : yins1;
       // the planes' slab rows, read while every lane is active (the lanes that
       // hold them lie in the ghost frame and store nothing)
       int xf[K], xre[K], xrh[K];
@@ -423,8 +583,8 @@ __device__ __forceinline__ void blocked_step_2d(const Slot<T>* __restrict__ slot
         }
         if (CLS != 1 && !yplain) {
           int dyes = 0, dyhs = 0, unused = 0;
-          const int syes = yins ? slab_e(js, jb, je, N, dyes, unused) : -1;
-          const int syhs = yins1 ? slab_h(js, jb, je, N, dyhs, unused) : -1;
+          const int syes = yins ? se(js, jb, je, dyes, unused) : -1;
+          const int syhs = yins1 ? sh(js, jb, je, dyhs, unused) : -1;
           T* opy = psiB[psi_id(R::PY, 1, 0)];
           T* oqy = psiB[psi_id(R::QY, 1, 0)];
           const unsigned oe = (unsigned)dyes * es + (syes == 1 ? s.psi_hi[1] : 0u);
@@ -432,19 +592,19 @@ __device__ __forceinline__ void blocked_step_2d(const Slot<T>* __restrict__ slot
 #pragma unroll
           for (int q = 0; q < K; ++q) {
             const int i = ib1 + q;
-            if (i < i0 || i >= i0 + TX || i < ib + (tm ? 0 : 1) || i >= ie) continue;
-            if (syes >= 0) stg<T>(opy, (unsigned)(i * N) * es + oe, py[q]);
-            if (syhs >= 0) stg<T>(oqy, (unsigned)(i * N) * es + oh, qy[q]);
+            if (i < i0 || i >= i0 + TX || i >= ie) continue;
+            if (syes >= 0 && i >= pye) stg<T>(opy, (unsigned)(i * N) * es + oe, py[q]);
+            if (syhs >= 0 && i >= pyh) stg<T>(oqy, (unsigned)(i * N) * es + oh, qy[q]);
           }
         }
-        if (kX && yxs) {
+        if (kX) {
 #pragma unroll
           for (int q = 0; q < K; ++q) {
             const int i = ib1 + q;
             if (i < i0 || i >= i0 + TX) continue;
-            if (xf[q] & 8)
+            if ((xf[q] & 8) && yxes)
               stg<T>(psiB[psi_id(R::PX, 0, xre[q] >= kHi)], (unsigned)((xre[q] & (kHi - 1)) * ny + js) * es, px[q]);
-            if (xf[q] & 16)
+            if ((xf[q] & 16) && yxhs)
               stg<T>(psiB[psi_id(R::QX, 0, xrh[q] >= kHi)], (unsigned)((xrh[q] & (kHi - 1)) * ny + js) * es, qx[q]);
           }
         }
@@ -467,13 +627,23 @@ __device__ __forceinline__ void blocked_step_2d(const Slot<T>* __restrict__ slot
 template <typename T, int TB, int W, int K, int MW>
 __global__ __launch_bounds__(64 * W, MW) void k_tmz_tb(const Slot<T>* __restrict__ slots,
                                                        const int4* __restrict__ tiles, int ntiles, int tstep) {
-  blocked_step_2d<T, SCHEME_TMZ, TB, W, K>(slots, tiles, ntiles, tstep);
+  blocked_step_2d<T, SCHEME_TMZ, TB, W, K, 0>(slots, tiles, ntiles, tstep, nullptr, nullptr);
 }
 
-template <typename T, int TB, int W, int K, int MW>
+template <typename T, int TB, int W, int K, int MW, int MON>
 __global__ __launch_bounds__(64 * W, MW) void k_tez_tb(const Slot<T>* __restrict__ slots,
-                                                       const int4* __restrict__ tiles, int ntiles, int tstep) {
-  blocked_step_2d<T, SCHEME_TEZ, TB, W, K>(slots, tiles, ntiles, tstep);
+                                                       const int4* __restrict__ tiles, int ntiles, int tstep,
+                                                       const Monitor<T>* __restrict__ mons,
+                                                       const int2* __restrict__ smon) {
+  blocked_step_2d<T, SCHEME_TEZ, TB, W, K, MON>(slots, tiles, ntiles, tstep, mons, smon);
+}
+
+template <typename T, int TB, int W, int K, int MW, int MON>
+__global__ __launch_bounds__(64 * W, MW) void k_tmzl_tb(const Slot<T>* __restrict__ slots,
+                                                        const int4* __restrict__ tiles, int ntiles, int tstep,
+                                                        const Monitor<T>* __restrict__ mons,
+                                                        const int2* __restrict__ smon) {
+  blocked_step_2d<T, SCHEME_TMZ_LOSSY, TB, W, K, MON>(slots, tiles, ntiles, tstep, mons, smon);
 }
 
 }  // namespace oidt

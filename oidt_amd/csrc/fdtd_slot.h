@@ -106,6 +106,7 @@ struct Monitor {
   int x0, y0, z0, ex, ey, ez;   // box origin and extent
   int gx, gy, gz;               // real grid extents: stencil points outside read 0
   int shift, nrec;
+  int after_h;   // 0: taken after the E half-step, 1: after the H half-step
 };
 
 }  // namespace oidt

@@ -455,7 +455,8 @@ def prepare(c, launch=(0, 0, 0)):
     s, fg, cb = build(c)
     sol = Solver.from_arrays(LossyTmArrays(c, fg), c.nt) if c.scheme == 'tm' else Solver(s, fg, cb=cb)
     try:
-        sol.set_launch(xchunk, grid, variant)
+        if variant or xchunk or grid:   # otherwise the library picks the form
+            sol.set_launch(xchunk, grid, variant)
         mons = monitors(c)
         ids = {k: sol.add_monitor(m) for k, m in mons.items()}
     except Exception:
@@ -489,7 +490,8 @@ def prepare_batch(cs, launch=(0, 0, 0)):
         raise ValueError('the study drivers need a two-kernel form (monitors sit between the half-steps)')
     b = Batch('tm_lossy' if scheme == 'tm' else scheme, np.float32, max_slots=len(cs))
     try:
-        b.set_launch(xchunk, grid, variant)
+        if variant or xchunk or grid:
+            b.set_launch(xchunk, grid, variant)
         runs = []
         for c in cs:
             s, fg, cb = build(c)

@@ -5,8 +5,8 @@ that come and go."""
 import numpy as np
 import pytest
 
-from oidt_amd import configs
-from oidt_amd.solver import Batch, Monitor
+from oidt_amd import configs, variants
+from oidt_amd.solver import Batch, Monitor, Solver
 
 from helpers import device_inputs, rel_l2
 
@@ -104,3 +104,35 @@ def test_form_changes_between_chunks(scheme):
     for x, y in zip(got_mon, b.read_monitor(k, i)):
         assert np.array_equal(x, y)
     b.close()
+
+
+# whole-plane and partial boxes, before and after the H half-step, records that
+# start late and end early, a batch small enough for the narrow tile and one
+# that is not
+@pytest.mark.gpu
+@pytest.mark.parametrize('scheme', ['te', 'tm'])
+@pytest.mark.parametrize('copies', [1, 9])
+def test_folded_monitors_match_monitor_kernel(scheme, copies):
+    names = ('ey', 'hz') if scheme == 'te' else ('hy', 'ez', 'hx')
+    over = dict(port1_length=1e-6) if scheme == 'te' else dict(port_length=1e-6)
+    cs = [variants.truncate(variants.config(scheme, 'scattering_loss', sgl_wg_length=6e-6, points_per_wl=20,
+                                            gauss_pulse_deg=-1, profile_number=k, **over), 75 + k) for k in range(copies)]
+    print('case', scheme, copies, cs[0].nx, cs[0].ny, flush=True)
+    out = []
+    for launch in ((2, 4, 0), (0, 0, 0)):
+        out.append(variants.run_batch(cs, launch))
+        c = cs[0]
+        rng = np.random.default_rng(3)
+        boxes = [[(0, c.nx), (0, c.ny)], [(17, 60), (40, 97)], [(c.nx - 33, c.nx), (c.ny - 1, c.ny)]]
+        s, fg, cb = variants.build(c)
+        sol = Solver.from_arrays(variants.LossyTmArrays(c, fg), c.nt) if scheme == 'tm' else Solver(s, fg, cb=cb)
+        if launch[0]:
+            sol.set_launch(launch[1], launch[2], launch[0])
+        ids = [sol.add_monitor(Monitor(n, [(0, 0)], 0.7, boxes[(k + 1) % 3], 50, after_h=bool(k & 1), shift=-11 + 6 * k,
+                                       cs=rng.standard_normal((50, 2)))) for k, n in enumerate(names)]
+        sol.run()
+        out[-1].append({(n, part): a for n, i in zip(names, ids) for part, a in enumerate(sol.read_monitor(i))})
+        sol.close()
+    for ref, got in zip(*out):
+        for k in ref:
+            assert np.array_equal(got[k], ref[k]), k
