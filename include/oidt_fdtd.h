@@ -162,6 +162,16 @@ int32_t oidt_chunk_steps(void);
  * Replaces fdtd_main.py:216-261 (cuda.to_device of every array). */
 int oidt_solver_create(const oidt_run_desc* desc, const oidt_run_inputs* in, oidt_solver** out);
 
+/* As oidt_solver_create / oidt_batch_add with the material given as one byte
+ * per cell ([nx][ny][nz]) instead of the cb maps: bits 2c..2c+1 of a byte index
+ * cb_values[c] (run precision, [3][4]) for E component c = 0..2 (Ex, Ey, Ez;
+ * lossy TMz: MOD_E in 0, CURL_H in 2).  in->cb is not read.  A two-material
+ * guide needs no maps of cb values then. */
+int oidt_solver_create_indexed(const oidt_run_desc* desc, const oidt_run_inputs* in, const uint8_t* material,
+                               const void* cb_values, oidt_solver** out);
+int oidt_batch_add_indexed(oidt_batch* b, const oidt_run_desc* desc, const oidt_run_inputs* in,
+                           const uint8_t* material, const void* cb_values, int32_t* slot);
+
 /* Launch knobs of a single run, as oidt_batch_set_launch; call before the
  * first oidt_solver_advance to change between fused and two-kernel forms.
  * No counterpart in the reference (fixed launch shapes, fdtd_main.py:263-273). */
@@ -183,6 +193,12 @@ int oidt_solver_steps(oidt_solver* s, int32_t* steps);
  * 0 = Ex, 1 = Ey, 2 = Hx, 3 = Hy (3D).  port: 0 or 1.
  * Replaces the copy_to_host calls of fdtd_main.py:349-357. */
 int oidt_solver_read_dft(oidt_solver* s, int32_t port, int32_t comp, double* re, double* im);
+
+/* The same phasors as complex pairs in the reference's full-plane layout:
+ * out is [nf][ny] (2D) or [nf][nx][ny] (3D) complex doubles, of which the
+ * window cells are written and the others left as they are.
+ * Replaces EZF1 = EZ1r + 1j*EZ1i of fdtd_main.py:359-363. */
+int oidt_solver_read_dft_plane(oidt_solver* s, int32_t port, int32_t comp, double* out);
 
 /* Copy one field component ([nx][ny][nz], run precision) to the host. */
 int oidt_solver_read_field(oidt_solver* s, int32_t field, void* host, uint64_t nbytes);
@@ -228,6 +244,7 @@ int oidt_batch_progress(oidt_batch* b, int64_t* chunks_enqueued, int64_t* chunks
 /* DFT of one slot (layout as oidt_solver_read_dft).  A run whose last chunk
  * has completed is read without waiting for the rest of the batch. */
 int oidt_batch_read_dft(oidt_batch* b, int32_t slot, int32_t port, int32_t comp, double* re, double* im);
+int oidt_batch_read_dft_plane(oidt_batch* b, int32_t slot, int32_t port, int32_t comp, double* out);
 int oidt_batch_read_field(oidt_batch* b, int32_t slot, int32_t field, void* host, uint64_t nbytes);
 
 /* Port power on the device, per frequency: the sum over rows [row0, row0 +

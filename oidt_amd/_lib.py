@@ -61,6 +61,12 @@ SIGNATURES = {
     'oidt_solver_sync': (C.c_int, [C.c_void_p]),
     'oidt_solver_steps': (C.c_int, [C.c_void_p, C.POINTER(C.c_int32)]),
     'oidt_solver_read_dft': (C.c_int, [C.c_void_p, C.c_int32, C.c_int32, C.c_void_p, C.c_void_p]),
+    'oidt_solver_read_dft_plane': (C.c_int, [C.c_void_p, C.c_int32, C.c_int32, C.c_void_p]),
+    'oidt_batch_read_dft_plane': (C.c_int, [C.c_void_p, C.c_int32, C.c_int32, C.c_int32, C.c_void_p]),
+    'oidt_solver_create_indexed': (C.c_int, [C.POINTER(RunDesc), C.POINTER(RunInputs), C.c_void_p, C.c_void_p,
+                                             C.POINTER(C.c_void_p)]),
+    'oidt_batch_add_indexed': (C.c_int, [C.c_void_p, C.POINTER(RunDesc), C.POINTER(RunInputs), C.c_void_p, C.c_void_p,
+                                         C.POINTER(C.c_int32)]),
     'oidt_solver_read_field': (C.c_int, [C.c_void_p, C.c_int32, C.c_void_p, C.c_uint64]),
     'oidt_solver_add_monitor': (C.c_int, [C.c_void_p, C.POINTER(MonitorDesc), C.POINTER(C.c_int32)]),
     'oidt_solver_read_monitor': (C.c_int, [C.c_void_p, C.c_int32, C.c_void_p, C.c_void_p, C.c_uint64]),

@@ -353,15 +353,18 @@ struct oidt_solver {
 namespace {
 
 // Device-memory image of one run, built on the host.
+// `material` / `values`: the material bytes and their cb values where the
+// caller has them already (oidt_batch_add_indexed), else null.
 template <typename T>
-int build_slot(oidt_batch* b, SlotHost& sh, const oidt_run_desc& d, const oidt_run_inputs* in) {
+int build_slot(oidt_batch* b, SlotHost& sh, const oidt_run_desc& d, const oidt_run_inputs* in,
+               const uint8_t* material, const void* values) {
   const Layout<T> L = layout<T>(d);
   const size_t cells = (size_t)d.nx * d.ny * d.nz;
   // maps per scheme and the material-byte component each is indexed under;
   // lossy TMz: {CURL_H, MOD_E}
   const int ncb = d.scheme == SCHEME_TMZ ? 1 : (d.scheme == SCHEME_3D ? 3 : 2);
   const int cb_comp[4][3] = {{2, -1, -1}, {0, 1, -1}, {0, 1, 2}, {2, 0, -1}};
-  for (int c = 0; c < ncb; ++c)
+  for (int c = 0; c < ncb && !material; ++c)
     if (!in->cb[c]) return fail(OIDT_EINVAL, "missing cb map");
   const int naxes = d.scheme == SCHEME_3D ? 3 : 2;
   for (int a = 0; a < naxes; ++a)
@@ -378,26 +381,43 @@ int build_slot(oidt_batch* b, SlotHost& sh, const oidt_run_desc& d, const oidt_r
   const size_t pcells = (size_t)pd.nx * pd.ny * pd.nz;
   std::vector<uint8_t> mat(pcells, 0);
   T cbv[3][kMatMax] = {};
-  for (int c = 0; c < ncb; ++c) {
+  if (material) {
+    for (size_t r = 0; r < cells / row; ++r) std::memcpy(&mat[r * prow], material + r * row, row);
+    std::memcpy(cbv, values, sizeof(cbv));
+  }
+  for (int c = 0; c < ncb && !material; ++c) {
     const int comp = cb_comp[d.scheme][c];
     const T* src = static_cast<const T*>(in->cb[c]);
     int nv = 0;
     T vals[kMatMax] = {};
     int last = -1;
-    for (size_t e = 0; e < cells; ++e) {
-      const T v = src[e];
+    auto index_of = [&](T v) {
+      if (last >= 0 && vals[last] == v) return last;
       int id = -1;
-      if (last >= 0 && vals[last] == v) id = last;
       for (int q = 0; id < 0 && q < nv; ++q)
         if (vals[q] == v) id = q;
-      if (id < 0) {
-        if (nv == kMatMax)
-          return fail(OIDT_EINVAL, "cb map of component " + std::to_string(comp) + " has more than 4 distinct values");
+      if (id < 0 && nv < kMatMax) {
         vals[nv] = v;
         id = nv++;
       }
-      last = id;
-      mat[e / row * prow + e % row] |= (uint8_t)(id << (2 * comp));
+      return last = id;
+    };
+    for (size_t r = 0; r < cells / row; ++r) {
+      const T* p = src + r * row;
+      uint8_t* out = &mat[r * prow];
+      // most rows hold one value
+      const T v0 = p[0];
+      int differ = 0;
+      for (size_t k = 1; k < row; ++k) differ |= p[k] != v0;
+      const size_t n = differ ? row : 1;
+      int id = 0;
+      for (size_t k = 0; k < n; ++k) {
+        id = index_of(p[k]);
+        if (id < 0)
+          return fail(OIDT_EINVAL, "cb map of component " + std::to_string(comp) + " has more than 4 distinct values");
+        out[k] |= (uint8_t)(id << (2 * comp));
+      }
+      for (size_t k = n; k < row; ++k) out[k] |= (uint8_t)(id << (2 * comp));
     }
     for (int q = 0; q < kMatMax; ++q) cbv[comp][q] = vals[q];
   }
@@ -1083,6 +1103,33 @@ int read_rows(oidt_batch* b, const char* src, size_t pitch, size_t row_len, size
   return rc == OIDT_OK && prev.id >= 0 ? drain(prev) : rc;
 }
 
+// Contiguous device memory to the host through pinned pieces on stream `st`:
+// put(piece, first byte, bytes) moves each piece to its place while the next
+// one is on its way.  (A copy straight into the caller's pageable array runs at
+// a few GB/s.)
+template <typename Put>
+int read_pieces(oidt_batch* b, hipStream_t st, const void* src, size_t bytes, Put&& put) {
+  struct Piece { int id; void* p; size_t at, n; };
+  Piece prev{-1, nullptr, 0, 0};
+  auto drain = [&](const Piece& pc) -> int {
+    HIP_TRY(hipEventSynchronize(b->staging.bufs[pc.id].ev));
+    put(static_cast<const char*>(pc.p), pc.at, pc.n);
+    b->staging.bufs[pc.id].pending = false;
+    return OIDT_OK;
+  };
+  int rc = OIDT_OK;
+  for (size_t at = 0; at < bytes && rc == OIDT_OK; at += kReadPiece) {
+    Piece pc{-1, nullptr, at, std::min(kReadPiece, bytes - at)};
+    pc.id = b->staging.get(pc.n, &pc.p, prev.id);
+    if (pc.id < 0) return fail(OIDT_ENOMEM, "pinned staging allocation failed");
+    HIP_TRY(hipMemcpyAsync(pc.p, static_cast<const char*>(src) + at, pc.n, hipMemcpyDeviceToHost, st));
+    if (b->staging.submit(pc.id, st) != 0) return fail(OIDT_EHIP, "event record failed");
+    if (prev.id >= 0) rc = drain(prev);
+    prev = pc;
+  }
+  return rc == OIDT_OK && prev.id >= 0 ? drain(prev) : rc;
+}
+
 // True once the GPU has completed every chunk the run needs (later chunks skip it).
 bool slot_finished(oidt_batch* b, const SlotHost& sh) {
   reap_marks(b);
@@ -1198,7 +1245,11 @@ int oidt_batch_create(int32_t scheme, int32_t precision, int32_t max_slots, oidt
   return OIDT_OK;
 }
 
-int oidt_batch_add(oidt_batch* b, const oidt_run_desc* desc, const oidt_run_inputs* in, int32_t* slot) {
+}  // extern "C"
+
+namespace {
+int add_run(oidt_batch* b, const oidt_run_desc* desc, const oidt_run_inputs* in, const uint8_t* material,
+            const void* values, int32_t* slot) {
   if (!b || !in || !slot) return fail(OIDT_EINVAL, "null argument");
   int rc = validate(desc);
   if (rc != OIDT_OK) return rc;
@@ -1211,7 +1262,8 @@ int oidt_batch_add(oidt_batch* b, const oidt_run_desc* desc, const oidt_run_inpu
   SlotHost& sh = b->slots[si];
   sh = SlotHost();
   sh.desc = *desc;
-  rc = b->precision == OIDT_F64 ? build_slot<double>(b, sh, *desc, in) : build_slot<float>(b, sh, *desc, in);
+  rc = b->precision == OIDT_F64 ? build_slot<double>(b, sh, *desc, in, material, values)
+                                   : build_slot<float>(b, sh, *desc, in, material, values);
   if (rc != OIDT_OK) {
     if (sh.dmem) (void)hipFreeAsync(sh.dmem, b->stream);
     sh = SlotHost();
@@ -1225,6 +1277,19 @@ int oidt_batch_add(oidt_batch* b, const oidt_run_desc* desc, const oidt_run_inpu
   b->dirty = true;
   *slot = si;
   return OIDT_OK;
+}
+}  // namespace
+
+extern "C" {
+
+int oidt_batch_add(oidt_batch* b, const oidt_run_desc* desc, const oidt_run_inputs* in, int32_t* slot) {
+  return add_run(b, desc, in, nullptr, nullptr, slot);
+}
+
+int oidt_batch_add_indexed(oidt_batch* b, const oidt_run_desc* desc, const oidt_run_inputs* in, const uint8_t* material,
+                           const void* cb_values, int32_t* slot) {
+  if (!material || !cb_values) return fail(OIDT_EINVAL, "null material index");
+  return add_run(b, desc, in, material, cb_values, slot);
 }
 
 int oidt_batch_set_launch(oidt_batch* b, int32_t xchunk, int32_t grid_blocks, int32_t variant) {
@@ -1330,29 +1395,67 @@ int oidt_batch_progress(oidt_batch* b, int64_t* chunks_enqueued, int64_t* chunks
   return OIDT_OK;
 }
 
+}  // extern "C"
+
+namespace {
+// Accumulators of one port component, [nf][wcells] (re, im) pairs, in pieces.
+// A finished run's accumulators are final while later chunks run for the
+// others: they are read on a stream of their own then, without waiting for
+// the batch stream.
+template <typename Put>
+int read_acc(oidt_batch* b, const SlotHost& sh, int32_t port, int32_t comp, Put&& put) {
+  const oidt_run_desc& d = sh.desc;
+  const size_t bytes = (size_t)d.nf * sh.wcells * 2 * sizeof(double);
+  const size_t off = d.precision == OIDT_F64 ? layout<double>(d).off_acc : layout<float>(d).off_acc;
+  hipStream_t st = b->stream;
+  if (slot_finished(b, sh) && b->chunks_done < b->chunks_enqueued) {
+    if (!b->aux) HIP_TRY(hipStreamCreateWithFlags(&b->aux, hipStreamNonBlocking));
+    st = b->aux;
+  }
+  return read_pieces(b, st, static_cast<char*>(sh.dmem) + off + (size_t)(port * (sh.nq / 2) + comp) * bytes, bytes,
+                     std::forward<Put>(put));
+}
+}  // namespace
+
+extern "C" {
+
 int oidt_batch_read_dft(oidt_batch* b, int32_t slot, int32_t port, int32_t comp, double* re, double* im) {
   int rc = slot_ok(b, slot);
   if (rc != OIDT_OK) return rc;
   const SlotHost& sh = b->slots[slot];
-  const int ncomp = sh.nq / 2;
-  if (port < 0 || port > 1 || comp < 0 || comp >= ncomp) return fail(OIDT_EINVAL, "bad port or component");
+  if (port < 0 || port > 1 || comp < 0 || comp >= sh.nq / 2) return fail(OIDT_EINVAL, "bad port or component");
   if (!re || !im) return fail(OIDT_EINVAL, "null output");
+  if ((size_t)sh.desc.nf * sh.wcells == 0) return OIDT_OK;
+  return read_acc(b, sh, port, comp, [&](const char* p, size_t at, size_t n) {
+    const double* v = reinterpret_cast<const double*>(p);
+    const size_t e0 = at / 16;
+    for (size_t e = 0; e < n / 16; ++e) {
+      re[e0 + e] = v[2 * e];
+      im[e0 + e] = v[2 * e + 1];
+    }
+  });
+}
+
+int oidt_batch_read_dft_plane(oidt_batch* b, int32_t slot, int32_t port, int32_t comp, double* out) {
+  int rc = slot_ok(b, slot);
+  if (rc != OIDT_OK) return rc;
+  const SlotHost& sh = b->slots[slot];
+  if (port < 0 || port > 1 || comp < 0 || comp >= sh.nq / 2) return fail(OIDT_EINVAL, "bad port or component");
+  if (!out) return fail(OIDT_EINVAL, "null output");
   const oidt_run_desc& d = sh.desc;
-  const size_t n = (size_t)d.nf * sh.wcells;
-  if (n == 0) return OIDT_OK;
-  const size_t off = d.precision == OIDT_F64 ? layout<double>(d).off_acc : layout<float>(d).off_acc;
-  const int q = port * ncomp + comp;
-  std::vector<double> buf(2 * n);
-  // A finished run's accumulators are final while later chunks run for the
-  // others: read without waiting for the batch stream.
-  if (!slot_finished(b, sh)) HIP_TRY(hipStreamSynchronize(b->stream));
-  HIP_TRY(hipMemcpy(buf.data(), static_cast<char*>(sh.dmem) + off + (size_t)q * n * 2 * sizeof(double),
-                    2 * n * sizeof(double), hipMemcpyDeviceToHost));
-  for (size_t e = 0; e < n; ++e) {
-    re[e] = buf[2 * e];
-    im[e] = buf[2 * e + 1];
-  }
-  return OIDT_OK;
+  if ((size_t)d.nf * sh.wcells == 0) return OIDT_OK;
+  // window rows [N, ny - N) of every (frequency, x in [N, nx - N) (3D))
+  const size_t N = d.num_cpml, len = sh.wyn, rows = sh.wcells / len;
+  const size_t xs = d.scheme == SCHEME_3D ? d.nx : 1, x0 = d.scheme == SCHEME_3D ? N : 0;
+  return read_acc(b, sh, port, comp, [&](const char* p, size_t at, size_t n) {
+    for (size_t e = at / 16, end = (at + n) / 16; e < end;) {
+      const size_t row = e / len, c = e - row * len, m = std::min(len - c, end - e);
+      const size_t f = row / rows, x = x0 + row % rows;
+      std::memcpy(out + 2 * ((f * xs + x) * d.ny + N + c), p, m * 16);
+      p += m * 16;
+      e += m;
+    }
+  });
 }
 
 int oidt_batch_port_power(oidt_batch* b, int32_t slot, int32_t port, int32_t sub_slot, int32_t sub_port,
@@ -1579,9 +1682,11 @@ int oidt_batch_read_monitor(oidt_batch* b, int32_t slot, int32_t monitor, void* 
   if (!re || (dft && !im)) return fail(OIDT_EINVAL, "null output");
   HIP_TRY(hipStreamSynchronize(b->stream));
   reap_marks(b);
-  HIP_TRY(hipMemcpy(re, mh.re, want, hipMemcpyDeviceToHost));
-  if (dft) HIP_TRY(hipMemcpy(im, mh.im, want, hipMemcpyDeviceToHost));
-  return OIDT_OK;
+  auto into = [](void* out) {
+    return [out](const char* p, size_t at, size_t n) { std::memcpy(static_cast<char*>(out) + at, p, n); };
+  };
+  if ((rc = read_pieces(b, b->stream, mh.re, want, into(re))) != OIDT_OK || !dft) return rc;
+  return read_pieces(b, b->stream, mh.im, want, into(im));
 }
 
 int oidt_batch_profile_all(oidt_batch* b, int32_t nchunks, double* out_ms6) {
@@ -1679,7 +1784,11 @@ int oidt_batch_destroy(oidt_batch* b) {
 
 // ---- single run = batch of one -------------------------------------------
 
-int oidt_solver_create(const oidt_run_desc* desc, const oidt_run_inputs* in, oidt_solver** out) {
+}  // extern "C"
+
+namespace {
+int create_solver(const oidt_run_desc* desc, const oidt_run_inputs* in, const uint8_t* material, const void* values,
+                  oidt_solver** out) {
   if (!out) return fail(OIDT_EINVAL, "null output");
   *out = nullptr;
   int rc = validate(desc);
@@ -1690,13 +1799,26 @@ int oidt_solver_create(const oidt_run_desc* desc, const oidt_run_inputs* in, oid
     delete s;
     return rc;
   }
-  if ((rc = oidt_batch_add(s->b, desc, in, &s->slot)) != OIDT_OK) {
+  if ((rc = add_run(s->b, desc, in, material, values, &s->slot)) != OIDT_OK) {
     oidt_batch_destroy(s->b);
     delete s;
     return rc;
   }
   *out = s;
   return OIDT_OK;
+}
+}  // namespace
+
+extern "C" {
+
+int oidt_solver_create(const oidt_run_desc* desc, const oidt_run_inputs* in, oidt_solver** out) {
+  return create_solver(desc, in, nullptr, nullptr, out);
+}
+
+int oidt_solver_create_indexed(const oidt_run_desc* desc, const oidt_run_inputs* in, const uint8_t* material,
+                               const void* cb_values, oidt_solver** out) {
+  if (!material || !cb_values) return fail(OIDT_EINVAL, "null material index");
+  return create_solver(desc, in, material, cb_values, out);
 }
 
 int oidt_solver_set_launch(oidt_solver* s, int32_t xchunk, int32_t grid_blocks, int32_t variant) {
@@ -1727,6 +1849,11 @@ int oidt_solver_steps(oidt_solver* s, int32_t* steps) {
 int oidt_solver_read_dft(oidt_solver* s, int32_t port, int32_t comp, double* re, double* im) {
   if (!s) return fail(OIDT_EINVAL, "null solver");
   return oidt_batch_read_dft(s->b, s->slot, port, comp, re, im);
+}
+
+int oidt_solver_read_dft_plane(oidt_solver* s, int32_t port, int32_t comp, double* out) {
+  if (!s) return fail(OIDT_EINVAL, "null solver");
+  return oidt_batch_read_dft_plane(s->b, s->slot, port, comp, out);
 }
 
 int oidt_solver_read_field(oidt_solver* s, int32_t field, void* host, uint64_t nbytes) {

@@ -95,3 +95,29 @@ def cb_maps(s, fg):
         prev[a] = slice(0, -1)
         arr[inner] = 0.5 * (eps_map[inner] + eps_map[tuple(prev)])
     return tuple(dt / arr for arr in avg)
+
+
+def material_index(s, fg):
+    """(bytes, values): the CB maps of ``cb_maps`` as one byte per cell, bits
+    2c..2c+1 indexing row c of ``values`` (E components Ex, Ey, Ez; run
+    precision, [3, 4]).  A guide of two materials has three values per
+    component: background, their average, core."""
+    P = s.precision
+    fg = np.ascontiguousarray(fg, dtype=bool).view(np.uint8)
+    bg, core = s.eps * 1.0, s.eps * s.eps_rel_fg
+    lut = P(s.delta_t) / np.array([bg, 0.5 * (bg + core), core], dtype=np.float64).astype(P)
+    values = np.zeros((3, 4), dtype=P)
+    values[:, :3] = lut
+    if s.scheme == 'tm':
+        return fg << 5, values   # component 2: index 0 or 2
+    index = fg * np.uint8(2 * (1 + 4) if s.scheme == 'te' else 2 * (1 + 4 + 16))
+    inner = tuple(slice(1, None) for _ in range(fg.ndim))
+    here = fg[inner]
+    acc = None
+    for a in range(2 if s.scheme == 'te' else 3):
+        prev = [slice(1, None)] * fg.ndim
+        prev[a] = slice(0, -1)
+        part = (here + fg[tuple(prev)]) << (2 * a)
+        acc = part if acc is None else acc + part
+    index[inner] = acc
+    return index, values

@@ -33,11 +33,23 @@ class RunArrays:
         o = s.offset
         dims = (s.nx, s.ny, s.nz) if s.scheme == '3d' else (s.nx, s.ny)
         self.kappa = [M.kappa_axes(n, s.num_cpml, o, g['KE'], g['KH'], s.delta_x, P) for n in dims]
-        self.cb = [np.ascontiguousarray(a, dtype=P) for a in (M.cb_maps(s, fg) if cb is None else cb)]
+        # the material as indexes unless cb maps are given or asked for
+        self._cb = None if cb is None else [np.ascontiguousarray(a, dtype=P) for a in cb]
+        self.material = M.material_index(s, fg) if cb is None else None
         self.jsrc = np.ascontiguousarray(s.J_SRC, dtype=P)
         self.freqs = np.ascontiguousarray(s.sparam_freqs, dtype=np.float64)
         self.db = P(float(s.delta_t) / s.mu)   # DB = delta_t / mu (fdtd_main.py:86), narrowed at launch
         self.src_field, self.src_box = source_box(s, direction, line)
+
+    @property
+    def cb(self):
+        """The CB maps.  Once asked for they are what the library reads."""
+        if self._cb is None:
+            index, values = self.material
+            comps = {'tm': (2,), 'te': (0, 1), '3d': (0, 1, 2)}[self.setup.scheme]
+            self._cb = [values[c][(index >> (2 * c)) & 3] for c in comps]
+            self.material = None
+        return self._cb
 
     def desc(self):
         s = self.setup
@@ -61,9 +73,14 @@ class RunArrays:
         return d
 
     def inputs(self):
-        r = _lib.RunInputs()
+        r = self.inputs_without_maps()
         for c, a in enumerate(self.cb):
             r.cb[c] = ptr(a)
+        return r
+
+    def inputs_without_maps(self):
+        """The inputs of the calls that take ``material`` instead of CB maps."""
+        r = _lib.RunInputs()
         for a, (ke, kh) in enumerate(self.kappa):
             r.kappa_e[a] = ptr(ke)
             r.kappa_h[a] = ptr(kh)
@@ -130,6 +147,30 @@ def _window_cells(s):
     return (wy[1] - wy[0]) * ((wx[1] - wx[0]) if wx else 1)
 
 
+def _create(arrays, desc):
+    """(handle, inputs) of a single run."""
+    h = C.c_void_p()
+    material = getattr(arrays, 'material', None)
+    r = arrays.inputs() if material is None else arrays.inputs_without_maps()
+    if material is None:
+        check(lib().oidt_solver_create(C.byref(desc), C.byref(r), C.byref(h)))
+    else:
+        check(lib().oidt_solver_create_indexed(C.byref(desc), C.byref(r), ptr(material[0]), ptr(material[1]),
+                                               C.byref(h)))
+    return h, r
+
+
+def _read_planes(s, read):
+    """{(component key, port): full-plane phasors} with read(port, comp, array)."""
+    nf = len(s.sparam_freqs)
+    out = {}
+    for p in (0, 1):
+        for c, k in enumerate(COMP_KEYS[s.scheme]):
+            out[(k, p + 1)] = np.zeros((nf, s.nx, s.ny) if s.scheme == '3d' else (nf, s.ny), dtype=np.complex128)
+            read(p, c, out[(k, p + 1)])
+    return out
+
+
 class Solver:
     """One run on the device (a batch of one inside the library)."""
 
@@ -137,10 +178,7 @@ class Solver:
         self.arrays = RunArrays(setup, fg, direction, line, cb)
         self.setup = setup
         self._desc = self.arrays.desc()
-        self._in = self.arrays.inputs()
-        h = C.c_void_p()
-        check(lib().oidt_solver_create(C.byref(self._desc), C.byref(self._in), C.byref(h)))
-        self.h = h
+        self.h, self._in = _create(self.arrays, self._desc)
 
     @classmethod
     def from_arrays(cls, arrays, nt, precision=np.float32, shape=None):
@@ -150,14 +188,11 @@ class Solver:
         self = cls.__new__(cls)
         self.arrays = arrays
         self._desc = arrays.desc()
-        self._in = arrays.inputs()
         d = self._desc
         self.setup = SimpleNamespace(nt=nt, precision=precision,
                                      shape=shape or ((d.nx, d.ny, d.nz) if d.nz > 1 else (d.nx, d.ny)),
                                      scheme=None, sparam_freqs=np.zeros(0))
-        h = C.c_void_p()
-        check(lib().oidt_solver_create(C.byref(self._desc), C.byref(self._in), C.byref(h)))
-        self.h = h
+        self.h, self._in = _create(self.arrays, self._desc)
         return self
 
     def set_launch(self, xchunk=0, grid_blocks=0, variant=0):
@@ -191,9 +226,8 @@ class Solver:
 
     def dft(self):
         """{(component key, port 1|2): complex [nf, ny] (2D) or [nf, nx, ny] (3D)}."""
-        keys = COMP_KEYS[self.setup.scheme]
-        raw = {(k, p + 1): self.read_dft(p, c) for p in (0, 1) for c, k in enumerate(keys)}
-        return expand_dft(self.setup, raw)
+        return _read_planes(self.setup,
+                            lambda p, c, a: check(lib().oidt_solver_read_dft_plane(self.h, p, c, ptr(a))))
 
     def field(self, name):
         s = self.setup
@@ -250,9 +284,15 @@ class Batch:
     def add_arrays(self, arrays, setup):
         """Add a run from any object with ``desc()`` / ``inputs()``; ``setup``
         describes it to the Python side (nt, precision, shape, frequencies)."""
-        d, r = arrays.desc(), arrays.inputs()
+        d = arrays.desc()
         slot = C.c_int32()
-        check(lib().oidt_batch_add(self.h, C.byref(d), C.byref(r), C.byref(slot)))
+        material = getattr(arrays, 'material', None)
+        r = arrays.inputs() if material is None else arrays.inputs_without_maps()
+        if material is None:
+            check(lib().oidt_batch_add(self.h, C.byref(d), C.byref(r), C.byref(slot)))
+        else:
+            check(lib().oidt_batch_add_indexed(self.h, C.byref(d), C.byref(r), ptr(material[0]), ptr(material[1]),
+                                               C.byref(slot)))
         self.runs[slot.value] = setup
         self.monitors = getattr(self, 'monitors', {})
         self.monitors[slot.value] = []
@@ -325,10 +365,8 @@ class Batch:
         return re + 1j * im
 
     def dft(self, slot):
-        s = self.runs[slot]
-        keys = COMP_KEYS[s.scheme]
-        raw = {(k, p + 1): self.read_dft(slot, p, c) for p in (0, 1) for c, k in enumerate(keys)}
-        return expand_dft(s, raw)
+        return _read_planes(self.runs[slot],
+                            lambda p, c, a: check(lib().oidt_batch_read_dft_plane(self.h, int(slot), p, c, ptr(a))))
 
     def field(self, slot, name):
         s = self.runs[slot]

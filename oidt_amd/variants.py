@@ -224,12 +224,16 @@ def lossy_tm_coefficients(c, fg):
     arithmetic is float64)."""
     f32 = np.float32
     dt, dx = f32(c.delta_t), f32(c.delta_x)
-    sigma = np.zeros((c.nx, c.ny), f32)
-    eps_mask = (c.eps * (c.eps_rel_fg * fg + 1 * ~fg)).astype(f32)
+    # CURL_H and MOD_E of the two materials (background, core; sigma = 0), placed by the mask
+    sigma = np.zeros(2, f32)
+    core = np.array([False, True])
+    eps_mask = (c.eps * (c.eps_rel_fg * core + 1 * ~core)).astype(f32)
     out = {'CURL_E': f32(float(dt) / (c.mu * float(dx)))}
     den = (dx * (f32(2) * eps_mask + sigma * dt)).astype(f32)
-    out['CURL_H'] = (f32(2 * float(dt)) / den).astype(f32)
-    out['MOD_E'] = ((f32(2) * eps_mask - sigma * dt) / (f32(2) * eps_mask + sigma * dt)).astype(f32)
+    curl_h = (f32(2 * float(dt)) / den).astype(f32)
+    mod_e = ((f32(2) * eps_mask - sigma * dt) / (f32(2) * eps_mask + sigma * dt)).astype(f32)
+    out['CURL_H'] = np.where(fg, curl_h[1], curl_h[0])
+    out['MOD_E'] = np.where(fg, mod_e[1], mod_e[0])
     N, R = c.num_cpml, c.cpml_range
     m_grade, m_alpha = 4, 1
     sigma_max = 1.2 * (0.8 * (m_grade + 1) / (float(c.eta) * float(dx)))
@@ -325,11 +329,14 @@ def _profiles(c, length):
 def te_cb_maps(c, fg):
     """CBX, CBY of FDTD_2D_TE/scattering_loss/fdtd_main.py:37-47: the float32
     EPS_MASK averaged with float32 sums, then delta_t / EPS."""
-    mask = (c.eps * (c.eps_rel_fg * fg + 1 * ~fg)).astype(np.float32)
-    ex, ey = mask.copy(), mask.copy()
-    ex[1:, 1:] = (mask[1:, 1:] + mask[:-1, 1:]) * np.float32(0.5)
-    ey[1:, 1:] = (mask[1:, 1:] + mask[1:, :-1]) * np.float32(0.5)
-    return c.delta_t / ex, c.delta_t / ey
+    bg, core = (c.eps * (c.eps_rel_fg * np.array([0, 1]) + np.array([1, 0]))).astype(np.float32)
+    lut = c.delta_t / np.array([bg, (bg + core) * np.float32(0.5), core], dtype=np.float32)
+    out = []
+    for prev in (fg[:-1, 1:], fg[1:, :-1]):   # the i - 1 and j - 1 neighbour
+        cb = np.where(fg, lut[2], lut[0])
+        cb[1:, 1:][fg[1:, 1:] != prev] = lut[1]
+        out.append(cb)
+    return tuple(out)
 
 
 def setup_of(c):
@@ -524,25 +531,32 @@ def run_batch(cs, launch=(0, 0, 0)):
         b.close()
 
 
+def _phasor(re, im):
+    """re + 1j*im as complex64 (the reference's arrays; no temporaries)."""
+    z = np.empty(re.shape, dtype=np.complex64)
+    z.real, z.imag = re, im
+    return z
+
+
 def _output(c, key, mon, val):
     if c.scheme == 'tm':
         if c.study == 'scattering_loss':
             re, im = val
             # dEZfr.copy_to_host() - 1j*dEZfi.copy_to_host()  (fdtd_main.py:260-262)
-            return (re - 1j * im.astype(np.complex64)).astype(np.complex64)[:, :, 0]
+            return _phasor(re, -im)[:, :, 0]
         return val.reshape(c.nt, c.ny)
     if c.scheme == 'te':
         if c.study == 'scattering_loss':
             re, im = val
             # dHZfr.copy_to_host() - 1j*dHZfi.copy_to_host()  (fdtd_main.py:265-266)
-            return (re - 1j * im.astype(np.complex64)).astype(np.complex64)[:, :, 0]
+            return _phasor(re, -im)[:, :, 0]
         return val.reshape(c.nt, c.ny)
     if c.study == 'scattering_loss':
         re, im = val
         full = np.zeros((c.nx, c.ny), dtype=np.complex64)
         (x0, x1), (y0, y1) = mon.box[0], mon.box[1]
         # EX1 = EX1r + 1j*EX1i over the zero-initialised [nx, ny] arrays (fdtd_main.py:424-435)
-        full[x0:x1, y0:y1] = (re + 1j * im.astype(np.complex64))[:, :, 0]
+        full[x0:x1, y0:y1] = _phasor(re, im)[:, :, 0]
         return full
     out = np.zeros((c.nt, c.nx), dtype=np.float32)
     out[:, :c.nx - 2] = val.reshape(c.nt, c.nx - 2)
