@@ -310,6 +310,7 @@ struct oidt_batch {
   hipGraphExec_t gexec = nullptr;
   bool dirty = true;
   int ntiles = 0, nwork = 0;
+  bool dft_wide = false;   // DFT work items of 128 cells (64 otherwise)
   int xchunk = 4;
   int grid_override = 0;
   // the 3D march loads its read-once values non-temporally: set when the
@@ -716,22 +717,24 @@ int rebuild_lists(oidt_batch* b) {
         for (int y0 = 0; y0 < d.ny; y0 += kBX) tiles.push_back(make_int4(si, x0, y0, 0));
     }
   }
-  // DFT work items: kFB frequencies each, fewer when the whole batch would
-  // otherwise have too few items to fill the GPU (a small single run: its
-  // fold is a serial chain per item).  Each frequency's sum is formed the
-  // same way whatever the grouping.
-  int fb = kFB;
-  auto items = [&](int f) {
+  // DFT work items: 128 cells x kFB frequencies each; fewer frequencies, then
+  // fewer cells, when the whole batch would otherwise have too few items to
+  // fill the GPU.  A cell's and frequency's sum is the same whatever the
+  // grouping.
+  int fb = kFB, cells = 128;
+  auto items = [&]() {
     size_t n = 0;
     for (const SlotHost& sh : b->slots)
-      if (sh.used) n += (size_t)sh.nq * ((sh.wcells + kThreads - 1) / kThreads) * ((sh.desc.nf + f - 1) / f);
+      if (sh.used) n += (size_t)sh.nq * ((sh.wcells + cells - 1) / cells) * ((sh.desc.nf + fb - 1) / fb);
     return n;
   };
-  while (fb > 1 && items(fb) < 1024) fb >>= 1;
+  while (fb > kFT && items() < 512) fb >>= 1;
+  if (items() < 512) cells = 64;
+  b->dft_wide = cells != 64;
   for (int si = 0; si < (int)b->slots.size(); ++si) {
     const SlotHost& sh = b->slots[si];
     if (!sh.used) continue;
-    const int cblocks = (sh.wcells + kThreads - 1) / kThreads;
+    const int cblocks = (sh.wcells + cells - 1) / cells;
     for (int q = 0; q < sh.nq; ++q)
       for (int cb = 0; cb < cblocks; ++cb)
         for (int f0 = 0; f0 < sh.desc.nf; f0 += fb) work.push_back(make_int4(si, q, cb, f0 | (fb << 16)));
@@ -932,8 +935,12 @@ void launch_stencil(oidt_batch* b, int gs, int tstep, bool e_half) {
 
 template <typename T>
 void launch_dft(oidt_batch* b, int gd) {
-  hipLaunchKernelGGL((k_dft<T>), dim3(gd), dim3(kThreads), 0, b->stream,
-                     static_cast<const Slot<T>*>(b->d_slots), b->d_work, b->d_counts);
+  const Slot<T>* sl = static_cast<const Slot<T>*>(b->d_slots);
+  if (b->nwork == 0) return;
+  if (b->dft_wide)
+    hipLaunchKernelGGL((k_dft<T, 2>), dim3(gd), dim3(kThreads), 0, b->stream, sl, b->d_work, b->nwork);
+  else
+    hipLaunchKernelGGL((k_dft<T, 1>), dim3(gd), dim3(kThreads), 0, b->stream, sl, b->d_work, b->nwork);
 }
 
 template <typename T>

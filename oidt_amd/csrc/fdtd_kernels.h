@@ -3001,31 +3001,44 @@ __device__ __forceinline__ int sample_taps(const Slot<T>& s, int q, int c, size_
   return 4;
 }
 
-// The chunk's samples smp[t], t < tv, of one cell (zero from tv on).  Every
-// step's values load without a branch (steps past tv read step tv - 1 and are
-// discarded), so all of them are in flight together.
+// One step's sample of a cell (K taps from `o`), `r` the step's planes.
 template <typename T, int K>
-__device__ __forceinline__ void gather_samples(const T* __restrict__ ring, size_t stride, const size_t (&o)[4],
-                                               int tv, T (&smp)[kChunk]) {
-#pragma unroll
-  for (int t = 0; t < kChunk; ++t) {
-    const T* r = ring + (size_t)min(t, tv - 1) * stride;
-    T v = r[o[0]];
-    if constexpr (K > 1) v = v + r[o[1]];
-    if constexpr (K > 2) v = (v + r[o[2]]) + r[o[3]];
-    if constexpr (K == 2) v = T(0.5) * v;
-    if constexpr (K == 4) v = T(0.25) * v;
-    smp[t] = t < tv ? v : T(0);
-  }
+__device__ __forceinline__ T sample_at(const T* __restrict__ r, const size_t (&o)[4]) {
+  T v = r[o[0]];
+  if constexpr (K > 1) v = v + r[o[1]];
+  if constexpr (K > 2) v = (v + r[o[2]]) + r[o[3]];
+  if constexpr (K == 2) v = T(0.5) * v;
+  if constexpr (K == 4) v = T(0.25) * v;
+  return v;
 }
 
-template <typename T>
+// The fold as an FP64 matrix product: acc[f, cell] += W[f, t] x smp[t, cell]
+// over the chunk's 32 steps, W the cosines and sines.  A wave takes 16 NC cells
+// and kFT = 8 frequencies at a time (16 rows: cos and sin), eight 16 x 16 x 4
+// matrix instructions per 16 cells.  One read of a lane's weights serves NC of
+// them; as vector FMAs each weight is read from LDS by every lane, and the
+// 128 B per clock of LDS returns bound the fold.  Row 4 v + g of a tile is
+// (frequency g + 4 (v / 2), cos for even v, sin for odd v): a lane's four
+// results, rows 4 v + lane / 16, are then the (re, im) pairs of two
+// frequencies.  A work item is 64 NC cells x up to kFB frequencies of one
+// component; NC = 1 where a batch has too few items to fill the GPU, else 2
+// (NC = 4 takes 204 registers and was slower: 21 and 37 us in the first two
+// cases).  The sum of a cell and frequency does not depend on the grouping.
+// us per chunk, vector FMAs / this: 1480 x 430 with 1001 frequencies 32 / 18,
+// 128 x 96 x 320 50 / 32, 97 x 65 x 193 FP64 88 / 21, 16 3D guides 244 / 194
+// (their accumulators, 876 MB read and written, take 170 at the copy rate).
+constexpr int kFT = 8;
+
+using double4v = double __attribute__((ext_vector_type(4)));
+
+template <typename T, int NC>
 __global__ __launch_bounds__(kThreads) void k_dft(const Slot<T>* __restrict__ slots,
-                                                  const int4* __restrict__ work,
-                                                  const int* __restrict__ counts) {
-  __shared__ double cs[kFB][kChunk];
-  __shared__ double sn[kFB][kChunk];
-  const int nwork = counts[1];
+                                                  const int4* __restrict__ work, int nwork) {
+  __shared__ double tab[2][kFB][kChunk + 1];   // cos, sin; rows one double apart in the banks
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int col = lane & 15, grp = lane >> 4;
+  // this lane's row of a weight tile
+  const int wf = (col & 3) + 4 * (col >> 3), wpart = (col >> 2) & 1;
   for (int ww = xcd_block(); ww < nwork; ww += gridDim.x) {
     const int4 wk = work[ww];
     const Slot<T>& s = slots[wk.x];
@@ -3037,70 +3050,78 @@ __global__ __launch_bounds__(kThreads) void k_dft(const Slot<T>* __restrict__ sl
     const bool hq = (s.scheme == SCHEME_3D) ? ((q & 3) >= 2) : ((q & 1) == 1);
     const double phi = hq ? 0.5 : 0.0;
     const int f0 = wk.w & 0xffff, fbn = wk.w >> 16;
-    // the samples load first (cells past the window read its last cell and
-    // fold nothing), in flight while the phase table is formed
-    const int c = wk.z * kThreads + threadIdx.x;
-    size_t o[4];
-    const int k = sample_taps(s, q, min(c, s.wcells - 1), o);
-    const size_t stride = (size_t)s.nplanes * s.pcells;
-    T smp[kChunk];
-    if (k == 1)
-      gather_samples<T, 1>(s.ring, stride, o, tv, smp);
-    else if (k == 2)
-      gather_samples<T, 2>(s.ring, stride, o, tv, smp);
-    else
-      gather_samples<T, 4>(s.ring, stride, o, tv, smp);
-    __syncthreads();
-    for (int e = threadIdx.x; e < fbn * kChunk; e += kThreads) {
-      const int fl = e / kChunk, t = e - fl * kChunk;
-      const int f = f0 + fl;
-      double cv = 0.0, sv = 0.0;
-      if (f < s.nf && t < tv) {
-        const double ph = (s.w[f] * ((double)(n0 + t) + phi)) * s.dt;
-        sincos(ph, &sv, &cv);
-      }
-      cs[fl][t] = cv;
-      sn[fl][t] = sv;
-    }
-    __syncthreads();
-    if (c >= s.wcells) continue;
     const int fend = min(fbn, s.nf - f0);
-    double* a = s.acc + (((size_t)q * s.nf + f0) * s.wcells + c) * 2;
-    const size_t fs = (size_t)s.wcells * 2;   // between frequencies
-    // four frequencies at a time: their accumulators load before the sums
-    int fl = 0;
-    for (; fl + 4 <= fend; fl += 4, a += 4 * fs) {
-      double ar[4], ai[4], re[4] = {0.0, 0.0, 0.0, 0.0}, im[4] = {0.0, 0.0, 0.0, 0.0};
+    const int wcells = s.wcells;
+    const size_t stride = (size_t)s.nplanes * s.pcells;
+    // ---- samples: lane (col, grp) holds steps 4 k + grp of cell c + col, in
+    // flight while the weights are formed (cells past the window read its last
+    // one and fold nothing; steps past the chunk's end are zero)
+    T smp[NC][kChunk / 4];
+    const int c0 = (wk.z * (kThreads / 64) + w) * 16 * NC;
+    auto gather = [&](auto taps) {
+      constexpr int K = decltype(taps)::value;
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        ar[u] = a[u * fs];
-        ai[u] = a[u * fs + 1];
-      }
+      for (int m = 0; m < NC; ++m) {
+        size_t o[4];
+        sample_taps(s, q, min(c0 + m * 16 + col, wcells - 1), o);
 #pragma unroll
-      for (int t = 0; t < kChunk; ++t) {
-        const double v = (double)smp[t];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          re[u] += v * cs[fl + u][t];
-          im[u] += v * sn[fl + u][t];
+        for (int k = 0; k < kChunk / 4; ++k) {
+          const int t = 4 * k + grp;
+          const T v = sample_at<T, K>(s.ring + (size_t)min(t, tv - 1) * stride, o);
+          smp[m][k] = t < tv ? v : T(0);
         }
       }
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        a[u * fs] = ar[u] + re[u];
-        a[u * fs + 1] = ai[u] - im[u];
-      }
+    };
+    {
+      size_t o[4];
+      const int k = sample_taps(s, q, 0, o);
+      if (k == 1) gather(std::integral_constant<int, 1>{});
+      else if (k == 2) gather(std::integral_constant<int, 2>{});
+      else gather(std::integral_constant<int, 4>{});
     }
-    for (; fl < fend; ++fl, a += fs) {
-      double re = 0.0, im = 0.0;
-#pragma unroll
-      for (int t = 0; t < kChunk; ++t) {
-        const double v = (double)smp[t];
-        re += v * cs[fl][t];
-        im += v * sn[fl][t];
+    __syncthreads();   // the previous item's weights are used up
+    const int frows = (fend + kFT - 1) / kFT * kFT;
+    for (int e = threadIdx.x; e < frows * kChunk; e += kThreads) {
+      const int fl = e / kChunk, t = e - fl * kChunk;
+      double cv = 0.0, sv = 0.0;
+      if (fl < fend && t < tv) {
+        const double ph = (s.w[f0 + fl] * ((double)(n0 + t) + phi)) * s.dt;
+        sincos(ph, &sv, &cv);
       }
-      a[0] += re;
-      a[1] -= im;
+      tab[0][fl][t] = cv;
+      tab[1][fl][t] = sv;
+    }
+    __syncthreads();
+    if (c0 >= wcells) continue;   // uniform over the wave; no barrier below
+    for (int fl = 0; fl < fend; fl += kFT) {
+      // accumulators of this lane's two frequencies, loaded before the sums
+      double2 a[NC][2];
+      bool ok[NC][2];
+      double* p[NC][2];
+#pragma unroll
+      for (int m = 0; m < NC; ++m)
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          const int f = fl + grp + 4 * u, c = c0 + m * 16 + col;
+          ok[m][u] = f < fend && c < wcells;
+          p[m][u] = s.acc + (((size_t)q * s.nf + f0 + (ok[m][u] ? f : 0)) * wcells + (ok[m][u] ? c : 0)) * 2;
+          a[m][u] = *reinterpret_cast<const double2*>(p[m][u]);
+        }
+      double4v d[NC];
+#pragma unroll
+      for (int m = 0; m < NC; ++m) d[m] = double4v{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+      for (int k = 0; k < kChunk / 4; ++k) {
+        const double wv = tab[wpart][fl + wf][4 * k + grp];
+#pragma unroll
+        for (int m = 0; m < NC; ++m)
+          d[m] = __builtin_amdgcn_mfma_f64_16x16x4f64(wv, (double)smp[m][k], d[m], 0, 0, 0);
+      }
+#pragma unroll
+      for (int m = 0; m < NC; ++m)
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+          if (ok[m][u]) *reinterpret_cast<double2*>(p[m][u]) = make_double2(a[m][u].x + d[m][2 * u], a[m][u].y - d[m][2 * u + 1]);
     }
   }
 }
