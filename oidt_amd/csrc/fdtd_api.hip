@@ -582,14 +582,35 @@ bool blocked2d_monitors(const oidt_batch* b) {
   return true;
 }
 
-// The form the launches use.  Where the caller has not set the launch knobs
-// (to keep them counts too), 2D runs whose field monitors it can fold take the blocked step at its largest depth: a field passes
-// through HBM once per 8 steps and the launches fall from 64 to 4 per chunk.
-// Two-kernel / blocked, us per step: 140 x 72 10.5 / 1.6, 600 x 240 FP64 11.1 /
-// 2.0, 1480 x 430 12.6 / 2.5, 64 guides of 800..4000 x 240 353 / 57.  It gives
-// the two-kernel form's bits, and at a chunk boundary every run's state is
-// back in field set A, so a batch may change between the two there (a
-// monitored run joins or leaves).
+// Bytes of the resident runs' fields.
+size_t field_bytes(const oidt_batch* b) {
+  size_t n = 0;
+  for (const SlotHost& sh : b->slots)
+    if (sh.used) n += (size_t)sh.desc.nx * sh.desc.ny * sh.desc.nz * 6 * (b->precision == OIDT_F64 ? 8 : 4);
+  return n;
+}
+constexpr size_t kCacheFields = (size_t)192 << 20;   // fields beyond this do not stay in the 256 MiB last-level cache
+
+// The form the launches use where the caller has not set the launch knobs (to
+// keep them counts as setting them).
+//
+// 2D runs whose field monitors it can fold take the blocked step at its
+// largest depth: a field passes through HBM once per 8 steps and the launches
+// fall from 64 to 4 per chunk.  Two-kernel / blocked, us per step: 140 x 72
+// 10.5 / 1.6, 600 x 240 FP64 11.1 / 2.0, 1480 x 430 12.6 / 2.5, 64 guides of
+// 800..4000 x 240 353 / 57.
+//
+// FP32 3D runs without monitors take the blocked step where their fields
+// exceed the last-level cache: the march is then bound by HBM.  March /
+// blocked, us per step: 4 guides of 128 x 96 x 320 (360 MiB) 271 / 252, 16 of
+// 64 x 48 x 193 (217) 254 / 177, 12 of 70 x 48 x 250 (230) 250 / 230, 16 of 110
+// x 70 x 400 983 / 659, 320 x 320 x 400 799 / 533; within the cache one 128 x
+// 96 x 320 (90) 61 / 86, 4 of 96 x 64 x 192..312 (141) 99 / 166.  In FP64 its
+// tiles own half the rows they step: 228 / 311 on those 4.
+//
+// The blocked steps give the two-kernel forms' bits in FP32, and at a chunk
+// boundary every run's state is back in field set A, so a batch may change
+// between the two there (a run joins or leaves).
 void resolve_form(oidt_batch* b) {
   b->run_variant = b->variant;
   b->run_xchunk = b->xchunk;
@@ -597,12 +618,20 @@ void resolve_form(oidt_batch* b) {
     b->run_variant = 4;
     b->run_xchunk = 8;
   }
-  // Its lanes address the high-side y psi from the low-side array by a 32-bit
-  // offset (three slabs in between): runs beyond that take the two-kernel form.
-  if (b->run_variant == 4 && b->scheme != SCHEME_3D)
+  if (b->auto_form && b->scheme == SCHEME_3D && b->precision == OIDT_F32 && !b->has_monitors() &&
+      field_bytes(b) > kCacheFields) {
+    b->run_variant = 4;
+    b->run_xchunk = 2;
+  }
+  // The blocked steps address by 32-bit offsets: in 2D the high-side y psi from
+  // the low-side array (three slabs in between), in 3D every array of a run
+  // from its first field.  Runs beyond that take the two-kernel form.
+  if (b->run_variant == 4)
     for (const auto& sh : b->slots)
-      if (sh.used && 3.0 * ((double)sh.desc.nx * sh.desc.num_cpml * (b->precision == OIDT_F64 ? 8 : 4) + 256.0) > 4294967295.0) {
-        b->run_variant = 2;
+      if (sh.used && (b->scheme == SCHEME_3D
+                          ? sh.bytes > 4294967295ull
+                          : 3.0 * ((double)sh.desc.nx * sh.desc.num_cpml * (b->precision == OIDT_F64 ? 8 : 4) + 256.0) > 4294967295.0)) {
+        b->run_variant = b->scheme == SCHEME_3D ? 1 : 2;
         b->run_xchunk = 4;
       }
   for (auto& sh : b->slots)
@@ -743,11 +772,7 @@ int rebuild_lists(oidt_batch* b) {
   // last-level cache: above 192 MB the march's read-once loads bypass it
   // (measured: 16 runs of 96 x 64 x nz, 856 MB, 7 % faster; one run of
   // 128 x 96 x 320, 94 MB, 12 % slower)
-  size_t field_bytes = 0;
-  for (const SlotHost& sh : b->slots)
-    if (sh.used)
-      field_bytes += (size_t)sh.desc.nx * sh.desc.ny * sh.desc.nz * 6 * (b->precision == OIDT_F64 ? 8 : 4);
-  b->stream_loads = field_bytes > ((size_t)192 << 20);
+  b->stream_loads = field_bytes(b) > kCacheFields;
   int rc;
   if ((rc = grow(b, &b->d_tiles, &b->tiles_cap, std::max<size_t>(tiles.size(), 1))) != OIDT_OK) return rc;
   if ((rc = grow(b, &b->d_work, &b->work_cap, std::max<size_t>(work.size(), 1))) != OIDT_OK) return rc;

@@ -43,31 +43,6 @@
 
 namespace oidt {
 
-__device__ __forceinline__ float fmadd(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
-__device__ __forceinline__ double fmadd(double a, double b, double c) { return __builtin_fma(a, b, c); }
-
-// The value of lane l+1 / l-1; lane 63 / 0 gets zero (a ghost lane of every
-// tile: its wrong neighbour is discarded with the frame).  Without a value to
-// keep in the edge lane the shift folds into the subtraction that uses it.
-__device__ __forceinline__ float lane_next(float v) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x130, 0xf, 0xf, true));
-}
-__device__ __forceinline__ float lane_prev(float v) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x138, 0xf, 0xf, true));
-}
-__device__ __forceinline__ double lane_next(double v) {
-  const long long b = __double_as_longlong(v);
-  const int lo = __builtin_amdgcn_update_dpp(0, (int)b, 0x130, 0xf, 0xf, true);
-  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), 0x130, 0xf, 0xf, true);
-  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
-}
-__device__ __forceinline__ double lane_prev(double v) {
-  const long long b = __double_as_longlong(v);
-  const int lo = __builtin_amdgcn_update_dpp(0, (int)b, 0x138, 0xf, 0xf, true);
-  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), 0x138, 0xf, 0xf, true);
-  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
-}
-
 // A uniform / per-lane value the compiler may not connect with its origin: what
 // is derived from it is formed again after a long stretch of code instead of
 // being kept in registers across it.

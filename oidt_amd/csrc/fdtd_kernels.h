@@ -2130,6 +2130,31 @@ __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+__device__ __forceinline__ float fmadd(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+__device__ __forceinline__ double fmadd(double a, double b, double c) { return __builtin_fma(a, b, c); }
+
+// The value of lane l+1 / l-1; lane 63 / 0 gets zero (a ghost lane of every
+// tile: its wrong neighbour is discarded with the frame).  Without a value to
+// keep in the edge lane the shift folds into the subtraction that uses it.
+__device__ __forceinline__ float lane_next(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x130, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float lane_prev(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x138, 0xf, 0xf, true));
+}
+__device__ __forceinline__ double lane_next(double v) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)b, 0x130, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), 0x130, 0xf, 0xf, true);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+__device__ __forceinline__ double lane_prev(double v) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)b, 0x138, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), 0x138, 0xf, 0xf, true);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+
 __device__ __forceinline__ float lane_down1(float v, float hi) {
   return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(hi), __float_as_int(v), 0x130, 0xf, 0xf, false));
 }
@@ -2518,9 +2543,22 @@ __global__ __launch_bounds__(kThreads, 4) void k_3d_halo(const Slot<T>* __restri
 // registers.  Each step moves the cells that depend on values outside the
 // tile one cell inwards from every side (E reads H at +1 and H reads E at -1
 // along each axis), so after TB steps the inner cells are exact.  The
-// per-cell arithmetic and update ranges are k_3d_e's and k_3d_h's.  The
-// launch reads field/psi set ((n0 / TB) & 1) and writes the inner cells'
-// state after its steps to the other set.
+// update ranges are k_3d_e's and k_3d_h's, and the arithmetic is written with
+// the fused multiply-adds these compile to at their default depth: in FP32 the
+// results are the same bits.  The launch reads field/psi set ((n0 / TB) & 1)
+// and writes the inner cells' state after its steps to the other set.
+//
+// What bounds it: instruction issue and its three barriers per plane (one
+// 16-wave block per CU: 4.5 us per plane and two steps, near enough the same
+// where every tile has a CU of its own).  Rows outside the y slabs in tiles
+// without z slab, source or capture take the curls alone on the planes outside
+// the x slabs.  The loads run two positions ahead of their use.  For that the
+// compiler has to know how many are in flight, so the fields and y psi are
+// loaded without a branch around them, and the material comes as a dword (a
+// byte's zero extension waited for its load, and with it for all the others).
+// us per step, the march / this: 16 guides of 96 x 64 x 192..512 685 / 530
+// (560 before the loads ran ahead), 16 of 110 x 70 x 400 983 / 659, 320 x 320 x
+// 400 799 / 533, 128 x 96 x 320 61 / 86.
 constexpr int kTb3Seg = 32;   // planes of a 3D blocked tile
 
 // One cell's state: fields, psi and material byte.
@@ -2560,7 +2598,13 @@ __global__ __launch_bounds__(64 * W) void k_3d_tb(const Slot<T>* __restrict__ sl
   static_assert(TB == 2 && TY > 0 && kTb3Seg + 2 * TB <= 64, "two steps per launch");
   constexpr unsigned es = sizeof(T);
   __shared__ T xh[TB][2][W][64];   // old Hx, Hz of each row at each step's plane
-  __shared__ T xe[2][2][W][64];    // new Ex, Ez of each row (alternate steps alternate halves)
+  // new Ex, Ez of each row (alternate steps alternate halves), row w at w + 1:
+  // the row below is then at the wave's own address
+  __shared__ T xe[2][2][W + 1][64];
+  // x-slab coefficients be, ce, bh, ch of plane xf + u and the source waveform
+  // of step n0 + u (read on slab and source planes only; every wave writes the
+  // same values, and a barrier lies before the first read)
+  __shared__ T xc[5][64];
   const int ntiles = counts[0];
   const int lane = threadIdx.x;
   const int w = wave_id();
@@ -2582,6 +2626,7 @@ __global__ __launch_bounds__(64 * W) void k_3d_tb(const Slot<T>* __restrict__ sl
     const int xf = max(x0 - TB, 0), xl = min(xo1 - 1 + TB, nx - 1);   // loaded planes [xf, xl]
     const unsigned pl = (unsigned)ny * nz;
     const unsigned jk = (unsigned)jc * nz + kc;
+    const unsigned msh = 8u * ((unsigned)kc & 3u);   // this z-cell's byte in its dword of material bytes (rows are padded to 128 B)
     // ---- row (wave-uniform) constants
     const bool jin = j >= jb && j < je, jin1 = j > jb && j < je;
     int dj = 0, cj = 0, djh = 0, cjh = 0;
@@ -2604,15 +2649,14 @@ __global__ __launch_bounds__(64 * W) void k_3d_tb(const Slot<T>* __restrict__ sl
     // z-slab psi offsets within a plane row (the row part is added per plane)
     const unsigned izk = (unsigned)dk * es + (sk == 1 ? s.psi_hi[2] : 0u);
     const unsigned izkh = (unsigned)dkh * es + (skh == 1 ? s.psi_hi[2] : 0u);
-    // sources: TE on Ey (E half-step), TM on Hy (start of the H half-step);
-    // lane t holds the waveform of step n0 + t
+    // sources: TE on Ey (E half-step), TM on Hy (start of the H half-step)
     const bool ksrc = k >= s.sz0 && k < s.sz1 && j >= s.sy0 && j < s.sy1;
-    const T lk_jv = s.src_field >= 0 && lane < nsteps ? s.jsrc[n0 + lane] : T(0);
+    xc[4][lane] = s.src_field >= 0 && lane < nsteps ? s.jsrc[n0 + lane] : T(0);
     // capture: E at k = port (planes cap*6 + 0/1; 6/7 when the ports coincide),
     // Hx/Hy at k = port (2/4, 8/10) and port + 1 (3/5, 9/11)
     const bool jcap = own && j >= s.wy0 && j <= s.wy1;
     const int port0 = s.port[0], port1 = s.port[1];
-    const unsigned lflags =
+    unsigned lflags =
         (kin ? L3_KIN : 0u) | (kin1 ? L3_KIN1 : 0u) | (s.src_field == F_EY && ksrc ? L3_SRCE : 0u) |
         (s.src_field == F_HY && ksrc ? L3_SRCH : 0u) | (own ? L3_OWN : 0u) | (sk >= 0 ? L3_SK : 0u) |
         (skh >= 0 ? L3_SKH : 0u) | (jcap && k == port0 ? L3_CAPE0 | L3_CAPA : 0u) |
@@ -2621,17 +2665,26 @@ __global__ __launch_bounds__(64 * W) void k_3d_tb(const Slot<T>* __restrict__ sl
     // some lane of the tile captures (wave-uniform)
     const bool tcap = __builtin_amdgcn_readfirstlane(__any((lflags & L3_CAP) != 0u)) != 0;
     const bool tsrc = s.src_field >= 0;
-    // ---- x-only coefficients: lane u holds plane xf + u
-    T lx_ik = T(0), lx_be = T(0), lx_ce = T(0), lx_ikh = T(0), lx_bh = T(0), lx_ch = T(0);
+    // bulk curls alone on every plane outside the x slabs: a row outside the y
+    // slabs, no z slab, source or capture in the tile
+    const bool bulkrow = jin1 && sj < 0 && sjh < 0 && !zs && !tcap &&
+                         __builtin_amdgcn_readfirstlane(__any((lflags & (L3_SRCE | L3_SRCH)) != 0u)) == 0;
+    // ---- 1/kappa along x: lane u holds plane xf + u
+    T lx_ik = T(0), lx_ikh = T(0);
     {
       const int ip = xf + lane;
+      T be = T(0), ce = T(0), bh = T(0), ch = T(0);
       if (ip <= xl) {
         int d = 0, ci = 0;
         lx_ik = s.ike[0][ip];
-        if (slab_e(ip, ib, ie, N, d, ci) >= 0) { lx_be = s.be[ci]; lx_ce = s.ceo[ci]; }
+        if (slab_e(ip, ib, ie, N, d, ci) >= 0) { be = s.be[ci]; ce = s.ceo[ci]; }
         lx_ikh = s.ikh[0][ip];
-        if (slab_h(ip, ib, ie, N, d, ci) >= 0) { lx_bh = s.bh[ci]; lx_ch = s.cho[ci]; }
+        if (slab_h(ip, ib, ie, N, d, ci) >= 0) { bh = s.bh[ci]; ch = s.cho[ci]; }
       }
+      xc[0][lane] = be;
+      xc[1][lane] = ce;
+      xc[2][lane] = bh;
+      xc[3][lane] = ch;
     }
 
     // Plane i's fields and material byte, and its psi values, from set A
@@ -2682,7 +2735,7 @@ __global__ __launch_bounds__(64 * W) void k_3d_tb(const Slot<T>* __restrict__ sl
       if (lane == 58) otab = (unsigned)s.prow;
       if (lane == 59) otab = (unsigned)s.nplanes;
     }
-    unsigned ot = otab;   // the copy the accesses read (made opaque once per position)
+    unsigned ot = opaque_vgpr(otab);   // the copy the accesses read (made opaque once per position)
     auto O = [&](int c) { return (unsigned)__builtin_amdgcn_readlane((int)ot, c); };
     const T* const rbT = reinterpret_cast<const T*>(rb);
     T* const rbW = const_cast<T*>(rbT);
@@ -2695,23 +2748,23 @@ __global__ __launch_bounds__(64 * W) void k_3d_tb(const Slot<T>* __restrict__ sl
       c.ey = ldg<T>(rbT, O(F_EY) + bo);
       c.ez = ldg<T>(rbT, O(F_EZ) + bo);
       c.hx = ldg<T>(rbT, O(F_HX) + bo);
-      c.m = ldg<uint8_t>(reinterpret_cast<const uint8_t*>(rb), O(12) + idx);
+      c.m = ldg<unsigned>(reinterpret_cast<const unsigned*>(rb), O(12) + (idx & ~3u));
     };
     auto load_q = [&](int i, unsigned lf, Cell3<T>& c) {
       int di = 0, ci = 0, dih = 0, cih = 0;
       const int si = slab_e(i, ib, ie, N, di, ci);
       const int sih = slab_h(i, ib, ie, N, dih, cih);
-      // outside its slab a z lane reads element 0 (one line for the wave)
-      const unsigned ix = si >= 0 ? ((unsigned)di * pl + jk) * es + (si == 1 ? xhi : 0u) : 0u;
-      const unsigned ixh = sih >= 0 ? ((unsigned)dih * pl + jk) * es + (sih == 1 ? xhi : 0u) : 0u;
+      const unsigned ix = ((unsigned)di * pl + jk) * es + (si == 1 ? xhi : 0u);
+      const unsigned ixh = ((unsigned)dih * pl + jk) * es + (sih == 1 ? xhi : 0u);
+      // outside its slab a row or z lane reads element 0 (one line for the
+      // wave) and multiplies it by zero coefficients (z) or not at all (y)
       const unsigned iy = sj >= 0 ? (((unsigned)i * N + dj) * nz + kc) * es : 0u;
       const unsigned iyh = sjh >= 0 ? (((unsigned)i * N + djh) * nz + kc) * es : 0u;
       const unsigned zrow = ((unsigned)i * ny + jc) * N * es;
       const unsigned iz = (lf & L3_SK) ? zrow + izk : 0u;
       const unsigned izh = (lf & L3_SKH) ? zrow + izkh : 0u;
-      // psi loads only where a slab can hold the cell (the plane, the row or
-      // the tile is uniform over the wave); elsewhere the values are zero
-      c.qyx = c.qzx = c.ryx = c.rzx = c.qxy = c.qzy = c.rxy = c.rzy = c.qxz = c.qyz = c.rxz = c.ryz = T(0);
+      // (the zeros end the registers' life in a buffer that takes no new values)
+      c.qyx = c.qzx = c.ryx = c.rzx = c.qxz = c.qyz = c.rxz = c.ryz = T(0);
       if (si >= 0) {
         c.qyx = ldg<T>(rbT, O(14) + ix);
         c.qzx = ldg<T>(rbT, O(15) + ix);
@@ -2720,20 +2773,16 @@ __global__ __launch_bounds__(64 * W) void k_3d_tb(const Slot<T>* __restrict__ sl
         c.ryx = ldg<T>(rbT, O(16) + ixh);
         c.rzx = ldg<T>(rbT, O(17) + ixh);
       }
-      if (sj >= 0) {
-        c.qxy = ldg<T>(rbT, O(18) + iy);
-        c.qzy = ldg<T>(rbT, O(19) + iy);
-      }
-      if (sjh >= 0) {
-        c.rxy = ldg<T>(rbT, O(20) + iyh);
-        c.rzy = ldg<T>(rbT, O(21) + iyh);
-      }
       if (zs) {
         c.qxz = ldg<T>(rbT, O(22) + iz);
         c.qyz = ldg<T>(rbT, O(23) + iz);
         c.rxz = ldg<T>(rbT, O(24) + izh);
         c.ryz = ldg<T>(rbT, O(25) + izh);
       }
+      c.qxy = ldg<T>(rbT, O(18) + iy);
+      c.qzy = ldg<T>(rbT, O(19) + iy);
+      c.rxy = ldg<T>(rbT, O(20) + iyh);
+      c.rzy = ldg<T>(rbT, O(21) + iyh);
     };
 
     // One Yee step of cell c (plane i, step n0 + st): E, then H.  hyn, hzn:
@@ -2748,44 +2797,49 @@ __global__ __launch_bounds__(64 * W) void k_3d_tb(const Slot<T>* __restrict__ sl
                          {s.cbv[2][0], s.cbv[2][1], s.cbv[2][2], s.cbv[2][3]}};
     auto cbc = [&](unsigned m, int c) -> T {
       if constexpr (sizeof(T) == 4) {
-        const int q = (m >> (2 * c)) & 3;
-        return __int_as_float(__builtin_amdgcn_ds_bpermute((40 + 4 * c + q) * 4, (int)ot));
+        const unsigned q = __builtin_amdgcn_ubfe(m, msh + 2 * c, 2);
+        return __int_as_float(__builtin_amdgcn_ds_bpermute((int)((40 + 4 * c + q) * 4), (int)ot));
       } else {
-        return cb_of(cbd[c][0], cbd[c][1], cbd[c][2], cbd[c][3], m, c);
+        return cb_of(cbd[c][0], cbd[c][1], cbd[c][2], cbd[c][3], m >> msh, c);
       }
     };
     auto step = [&](Cell3<T>& c, int i, int st, unsigned lf, T hyn, T hzn, T hxu, T hzu, T& pey, T& pez) {
       const int u = i - xf;
-      const T ikx = lane_get(lx_ik, u), bex = lane_get(lx_be, u), cex = lane_get(lx_ce, u);
-      const T ikxh = lane_get(lx_ikh, u), bhx = lane_get(lx_bh, u), chx = lane_get(lx_ch, u);
+      const T ikx = lane_get(lx_ik, u), ikxh = lane_get(lx_ikh, u);
       const bool iin = i >= ib && i < ie, iin1 = i > ib && i < ie;
       const bool si = i >= ib && (i < ib + N || i >= ie - N) && i < ie;          // in an E x slab
       const bool sih = i > ib && (i < ib + N || i > ie - N) && i < ie;           // in an H x slab
       const bool lkin = (lf & L3_KIN) != 0u, lkin1 = (lf & L3_KIN1) != 0u;
       // ---- E (k_3d_e per cell)
-      const T hxk = lane_down1(c.hx, c.hx);
-      const T hyk = lane_down1(c.hy, c.hy);
+      const T hxk = lane_next(c.hx), hyk = lane_next(c.hy);   // lane 63 is a ghost cell
       T vx = c.ex, vy = c.ey, vz = c.ez;
+      const bool bulk = bulkrow && i >= ib + N && i < ie - N;
+      if (bulk) {
+        vx = fmadd(cbc(c.m, 0), fmadd(hzu - c.hz, iky, -((hyk - c.hy) * ikz)), vx);
+        vy = fmadd(cbc(c.m, 1), fmadd(hxk - c.hx, ikz, -((hzn - c.hz) * ikx)), vy);
+        vz = fmadd(cbc(c.m, 2), fmadd(hyn - c.hy, ikx, -((hxu - c.hx) * iky)), vz);
+      }
+      const bool srcx = !bulk && tsrc && i >= (int)O(52) && i < (int)O(53);
+      const T jv = srcx ? xc[4][st] : T(0);
+      if (!bulk) {
       if (iin1 && jin) {
         const T cb = cbc(c.m, 0);
         const T dHz = hzu - c.hz;
         const T dHy = hyk - c.hy;
-        T v = vx + cb * (dHz * iky - dHy * ikz);
-        if (sj >= 0) { const T qv = bej * c.qxy + cej * dHz; c.qxy = qv; v += cb * qv; }
-        if (zs) { const T qv = bek * c.qxz + cek * dHy; c.qxz = qv; v -= cb * qv; }
+        T v = fmadd(cb, fmadd(dHz, iky, -(dHy * ikz)), vx);
+        if (sj >= 0) { const T qv = fmadd(cej, dHz, bej * c.qxy); c.qxy = qv; v = fmadd(cb, qv, v); }
+        if (zs) { const T qv = fmadd(cek, dHy, bek * c.qxz); c.qxz = qv; v = fmadd(-cb, qv, v); }
         vx = lkin ? v : vx;
       }
-      const bool srcx = tsrc && i >= (int)O(52) && i < (int)O(53);
       const bool srcp = srcx && (lf & L3_SRCE) != 0u;
-      const T jv = tsrc ? lane_get(lk_jv, st) : T(0);
       if (iin && jin1) {
         const T cb = cbc(c.m, 1);
         const T dHx = hxk - c.hx;
         const T dHz = hzn - c.hz;
-        T v = vy + cb * (dHx * ikz - dHz * ikx);
+        T v = fmadd(cb, fmadd(dHx, ikz, -(dHz * ikx)), vy);
         v = srcp ? v - jv : v;
-        if (si) { const T qv = bex * c.qyx + cex * dHz; c.qyx = qv; v -= cb * qv; }
-        if (zs) { const T qv = bek * c.qyz + cek * dHx; c.qyz = qv; v += cb * qv; }
+        if (si) { const T qv = fmadd(xc[0][u], c.qyx, xc[1][u] * dHz); c.qyx = qv; v = fmadd(-cb, qv, v); }
+        if (zs) { const T qv = fmadd(cek, dHx, bek * c.qyz); c.qyz = qv; v = fmadd(cb, qv, v); }
         vy = lkin ? v : (srcp ? vy - jv : vy);
       } else {
         vy = srcp ? vy - jv : vy;
@@ -2794,15 +2848,16 @@ __global__ __launch_bounds__(64 * W) void k_3d_tb(const Slot<T>* __restrict__ sl
         const T cb = cbc(c.m, 2);
         const T dHy = hyn - c.hy;
         const T dHx = hxu - c.hx;
-        T v = vz + cb * (dHy * ikx - dHx * iky);
-        if (si) { const T qv = bex * c.qzx + cex * dHy; c.qzx = qv; v += cb * qv; }
-        if (sj >= 0) { const T qv = bej * c.qzy + cej * dHx; c.qzy = qv; v -= cb * qv; }
+        T v = fmadd(cb, fmadd(dHy, ikx, -(dHx * iky)), vz);
+        if (si) { const T qv = fmadd(xc[0][u], c.qzx, xc[1][u] * dHy); c.qzx = qv; v = fmadd(cb, qv, v); }
+        if (sj >= 0) { const T qv = fmadd(cej, dHx, bej * c.qzy); c.qzy = qv; v = fmadd(-cb, qv, v); }
         vz = lkin1 ? v : vz;
+      }
       }
       c.ex = vx;
       c.ey = vy;
       c.ez = vz;
-      const bool capx = tcap && i >= x0 && i < xo1 && i >= (int)O(54) && i <= (int)O(55);
+      const bool capx = !bulk && tcap && i >= x0 && i < xo1 && i >= (int)O(54) && i <= (int)O(55);
       auto put = [&](T v, unsigned plane) {
         const unsigned rbase = (unsigned)(tstep + st) * O(59);
         const unsigned cw = (unsigned)(i - (int)O(54)) * O(58) + (unsigned)(j - (int)O(56));
@@ -2815,40 +2870,45 @@ __global__ __launch_bounds__(64 * W) void k_3d_tb(const Slot<T>* __restrict__ sl
       // ---- new Ex, Ez of row j - 1 from the wave below
       T* const xa = &xe[st & 1][0][0][0];
       T* const xb = &xe[st & 1][1][0][0];
-      xa[w * 64 + lane] = vx;
-      xb[w * 64 + lane] = vz;
+      xa[w * 64 + lane + 64] = vx;
+      xb[w * 64 + lane + 64] = vz;
       lds_barrier();
-      const T exm = w > 0 ? xa[(w - 1) * 64 + lane] : vx;
-      const T ezm = w > 0 ? xb[(w - 1) * 64 + lane] : vz;
+      const T exm = w > 0 ? xa[w * 64 + lane] : vx;
+      const T ezm = w > 0 ? xb[w * 64 + lane] : vz;
       // ---- H (k_3d_h per cell)
-      const T exk = lane_up1(vx, vx), eyk = lane_up1(vy, vy);
-      T hx = c.hx;
+      const T exk = lane_prev(vx), eyk = lane_prev(vy);   // lane 0 is a ghost cell
+      T hx = c.hx, hy = c.hy, hz = c.hz;
+      if (bulk) {
+        hx = fmadd(db, fmadd(vy - eyk, ikzh, -((vz - ezm) * ikyh)), hx);
+        hy = fmadd(db, fmadd(vz - pez, ikxh, -((vx - exk) * ikzh)), hy);
+        hz = fmadd(db, fmadd(vx - exm, ikyh, -((vy - pey) * ikxh)), hz);
+      } else {
       if (iin && jin1) {
         const T dEy = vy - eyk;
         const T dEz = vz - ezm;
-        T v = hx + db * (dEy * ikzh - dEz * ikyh);
-        if (sjh >= 0) { const T qv = bhj * c.rxy + chj * dEz; c.rxy = qv; v -= db * qv; }
-        if (zs) { const T qv = bhk * c.rxz + chk * dEy; c.rxz = qv; v += db * qv; }
+        T v = fmadd(db, fmadd(dEy, ikzh, -(dEz * ikyh)), hx);
+        if (sjh >= 0) { const T qv = fmadd(bhj, c.rxy, chj * dEz); c.rxy = qv; v = fmadd(-db, qv, v); }
+        if (zs) { const T qv = fmadd(bhk, c.rxz, chk * dEy); c.rxz = qv; v = fmadd(db, qv, v); }
         hx = lkin1 ? v : hx;
       }
       const bool srch = srcx && (lf & L3_SRCH) != 0u;
-      T hy = srch ? c.hy - jv : c.hy;
+      hy = srch ? c.hy - jv : c.hy;
       if (iin1 && jin) {
         const T dEz = vz - pez;
         const T dEx = vx - exk;
-        T v = hy + db * (dEz * ikxh - dEx * ikzh);
-        if (sih) { const T qv = bhx * c.ryx + chx * dEz; c.ryx = qv; v += db * qv; }
-        if (zs) { const T qv = bhk * c.ryz + chk * dEx; c.ryz = qv; v -= db * qv; }
+        T v = fmadd(db, fmadd(dEz, ikxh, -(dEx * ikzh)), hy);
+        if (sih) { const T qv = fmadd(xc[2][u], c.ryx, xc[3][u] * dEz); c.ryx = qv; v = fmadd(db, qv, v); }
+        if (zs) { const T qv = fmadd(bhk, c.ryz, chk * dEx); c.ryz = qv; v = fmadd(-db, qv, v); }
         hy = lkin1 ? v : hy;
       }
-      T hz = c.hz;
       if (iin1 && jin1) {
         const T dEx = vx - exm;
         const T dEy = vy - pey;
-        T v = hz + db * (dEx * ikyh - dEy * ikxh);
-        if (sih) { const T qv = bhx * c.rzx + chx * dEy; c.rzx = qv; v -= db * qv; }
-        if (sjh >= 0) { const T qv = bhj * c.rzy + chj * dEx; c.rzy = qv; v += db * qv; }
+        T v = fmadd(db, fmadd(dEx, ikyh, -(dEy * ikxh)), hz);
+        if (sih) { const T qv = fmadd(xc[2][u], c.rzx, xc[3][u] * dEy); c.rzx = qv; v = fmadd(-db, qv, v); }
+        if (sjh >= 0) { const T qv = fmadd(bhj, c.rzy, chj * dEx); c.rzy = qv; v = fmadd(db, qv, v); }
         hz = lkin ? v : hz;
+      }
       }
       c.hx = hx;
       c.hy = hy;
@@ -2873,6 +2933,7 @@ __global__ __launch_bounds__(64 * W) void k_3d_tb(const Slot<T>* __restrict__ sl
       stg_nt<T>(rbW, O(6 + F_HX) + bo, c.hx);
       stg_nt<T>(rbW, O(6 + F_HY) + bo, c.hy);
       stg_nt<T>(rbW, O(6 + F_HZ) + bo, c.hz);
+      if (bulkrow && i >= ib + N && i < ie - N) return;
       const bool iin = i >= ib && i < ie, iin1 = i > ib && i < ie;
       const bool lkin = (lf & L3_KIN) != 0u, lkin1 = (lf & L3_KIN1) != 0u;
       int di = 0, ci = 0, dih = 0, cih = 0;
@@ -2920,16 +2981,16 @@ __global__ __launch_bounds__(64 * W) void k_3d_tb(const Slot<T>* __restrict__ sl
     T pey[TB], pez[TB];
 #pragma unroll
     for (int st = 0; st < TB; ++st) pey[st] = pez[st] = T(0);
-    auto position = [&](int p, Cell3<T>& ld, const Cell3<T>& n1, Cell3<T>& c0, Cell3<T>& c1) {
-      const unsigned lf = opaque_vgpr(lflags);
-      ot = opaque_vgpr(otab);
-      // rows outside the grid (ghost rows of the edge tiles) load nothing:
-      // no updated cell reads them (E rows end below ny - 1, H rows start
-      // above row 0), and their stale values only reach such cells
-      if (p <= xl && jgrid) {
-        load_f(p, ld);
-        load_q(p, lf, ld);
-      }
+    auto position = [&](int p, Cell3<T>& ld, Cell3<T>& n1, Cell3<T>& c0, Cell3<T>& c1) {
+      const unsigned lf = lflags = opaque_vgpr(lflags);
+      ot = opaque_vgpr(ot);
+      // Loaded without a branch around it (planes past the last, and rows
+      // outside the grid, load the nearest one inside: no updated cell reads
+      // them, E rows end below ny - 1 and H rows start above row 0).
+      // The psi values follow one position later: they then live in three of
+      // the four buffers.
+      load_q(min(max(p - 1, xf), xl), lf, n1);
+      load_f(min(p, xl), ld);
       // old Hx, Hz of both steps' planes for the wave below
       xh[0][0][w][lane] = c0.hx;
       xh[0][1][w][lane] = c0.hz;
@@ -2950,6 +3011,8 @@ __global__ __launch_bounds__(64 * W) void k_3d_tb(const Slot<T>* __restrict__ sl
       // plane p - 3 is final
       if (p - 3 >= x0 && p - 3 < xo1 && (lf & L3_OWN)) store(c1, p - 3, lf);
     };
+    lflags = opaque_vgpr(lflags);
+    __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0): no load from before the march is waited for inside it
     Cell3<T> b0{}, b1{}, b2{}, b3{};
     const int pend = xo1 + TB;
     for (int p = xf; p <= pend; p += 4) {
