@@ -51,6 +51,10 @@ class RunArrays:
             self.material = None
         return self._cb
 
+    @cb.setter
+    def cb(self, maps):
+        self._cb, self.material = maps, None
+
     def desc(self):
         s = self.setup
         d = _lib.RunDesc()
