@@ -2550,15 +2550,17 @@ __global__ __launch_bounds__(kThreads, 4) void k_3d_halo(const Slot<T>* __restri
 //
 // What bounds it: instruction issue and its three barriers per plane (one
 // 16-wave block per CU: 4.5 us per plane and two steps, near enough the same
-// where every tile has a CU of its own).  Rows outside the y slabs in tiles
-// without z slab, source or capture take the curls alone on the planes outside
-// the x slabs.  The loads run two positions ahead of their use.  For that the
+// where every tile has a CU of its own).  Rows inside every update range, in
+// tiles without z slab, source or capture, take a body without selects inside
+// the x limits, with the x and y psi terms behind uniform branches.  The loads
+// run two positions ahead of their use.  For that the
 // compiler has to know how many are in flight, so the fields and y psi are
 // loaded without a branch around them, and the material comes as a dword (a
 // byte's zero extension waited for its load, and with it for all the others).
-// us per step, the march / this: 16 guides of 96 x 64 x 192..512 685 / 530
-// (560 before the loads ran ahead), 16 of 110 x 70 x 400 983 / 659, 320 x 320 x
-// 400 799 / 533, 128 x 96 x 320 61 / 86.
+// us per step, the march / this: 16 guides of 96 x 64 x 192..512 691 / 523
+// (560 before the loads ran ahead, 530 with the select-free body on the planes
+// and rows without psi only), 16 of 110 x 70 x 400 985 / 626, 320 x 320 x
+// 400 801 / 509, 128 x 96 x 320 61 / 86.
 constexpr int kTb3Seg = 32;   // planes of a 3D blocked tile
 
 // One cell's state: fields, psi and material byte.
@@ -2665,10 +2667,10 @@ __global__ __launch_bounds__(64 * W) void k_3d_tb(const Slot<T>* __restrict__ sl
     // some lane of the tile captures (wave-uniform)
     const bool tcap = __builtin_amdgcn_readfirstlane(__any((lflags & L3_CAP) != 0u)) != 0;
     const bool tsrc = s.src_field >= 0;
-    // bulk curls alone on every plane outside the x slabs: a row outside the y
-    // slabs, no z slab, source or capture in the tile
-    const bool bulkrow = jin1 && sj < 0 && sjh < 0 && !zs && !tcap &&
-                         __builtin_amdgcn_readfirstlane(__any((lflags & (L3_SRCE | L3_SRCH)) != 0u)) == 0;
+    // a row inside every update range, without z slab, source or capture in the
+    // tile: inside the x limits all its cells take the same terms
+    const bool lean = jin1 && !zs && !tcap &&
+                      __builtin_amdgcn_readfirstlane(__any((lflags & (L3_SRCE | L3_SRCH)) != 0u)) == 0;
     // ---- 1/kappa along x: lane u holds plane xf + u
     T lx_ik = T(0), lx_ikh = T(0);
     {
@@ -2813,11 +2815,24 @@ __global__ __launch_bounds__(64 * W) void k_3d_tb(const Slot<T>* __restrict__ sl
       // ---- E (k_3d_e per cell)
       const T hxk = lane_next(c.hx), hyk = lane_next(c.hy);   // lane 63 is a ghost cell
       T vx = c.ex, vy = c.ey, vz = c.ez;
-      const bool bulk = bulkrow && i >= ib + N && i < ie - N;
+      const bool bulk = lean && iin1;
       if (bulk) {
-        vx = fmadd(cbc(c.m, 0), fmadd(hzu - c.hz, iky, -((hyk - c.hy) * ikz)), vx);
-        vy = fmadd(cbc(c.m, 1), fmadd(hxk - c.hx, ikz, -((hzn - c.hz) * ikx)), vy);
-        vz = fmadd(cbc(c.m, 2), fmadd(hyn - c.hy, ikx, -((hxu - c.hx) * iky)), vz);
+        const T cbx = cbc(c.m, 0), cby = cbc(c.m, 1), cbz = cbc(c.m, 2);
+        vx = fmadd(cbx, fmadd(hzu - c.hz, iky, -((hyk - c.hy) * ikz)), vx);
+        vy = fmadd(cby, fmadd(hxk - c.hx, ikz, -((hzn - c.hz) * ikx)), vy);
+        vz = fmadd(cbz, fmadd(hyn - c.hy, ikx, -((hxu - c.hx) * iky)), vz);
+        if (si) {
+          c.qyx = fmadd(xc[0][u], c.qyx, xc[1][u] * (hzn - c.hz));
+          vy = fmadd(-cby, c.qyx, vy);
+          c.qzx = fmadd(xc[0][u], c.qzx, xc[1][u] * (hyn - c.hy));
+          vz = fmadd(cbz, c.qzx, vz);
+        }
+        if (sj >= 0) {
+          c.qxy = fmadd(cej, hzu - c.hz, bej * c.qxy);
+          vx = fmadd(cbx, c.qxy, vx);
+          c.qzy = fmadd(cej, hxu - c.hx, bej * c.qzy);
+          vz = fmadd(-cbz, c.qzy, vz);
+        }
       }
       const bool srcx = !bulk && tsrc && i >= (int)O(52) && i < (int)O(53);
       const T jv = srcx ? xc[4][st] : T(0);
@@ -2882,6 +2897,18 @@ __global__ __launch_bounds__(64 * W) void k_3d_tb(const Slot<T>* __restrict__ sl
         hx = fmadd(db, fmadd(vy - eyk, ikzh, -((vz - ezm) * ikyh)), hx);
         hy = fmadd(db, fmadd(vz - pez, ikxh, -((vx - exk) * ikzh)), hy);
         hz = fmadd(db, fmadd(vx - exm, ikyh, -((vy - pey) * ikxh)), hz);
+        if (sih) {
+          c.ryx = fmadd(xc[2][u], c.ryx, xc[3][u] * (vz - pez));
+          hy = fmadd(db, c.ryx, hy);
+          c.rzx = fmadd(xc[2][u], c.rzx, xc[3][u] * (vy - pey));
+          hz = fmadd(-db, c.rzx, hz);
+        }
+        if (sjh >= 0) {
+          c.rxy = fmadd(bhj, c.rxy, chj * (vz - ezm));
+          hx = fmadd(-db, c.rxy, hx);
+          c.rzy = fmadd(bhj, c.rzy, chj * (vx - exm));
+          hz = fmadd(db, c.rzy, hz);
+        }
       } else {
       if (iin && jin1) {
         const T dEy = vy - eyk;
@@ -2933,7 +2960,7 @@ __global__ __launch_bounds__(64 * W) void k_3d_tb(const Slot<T>* __restrict__ sl
       stg_nt<T>(rbW, O(6 + F_HX) + bo, c.hx);
       stg_nt<T>(rbW, O(6 + F_HY) + bo, c.hy);
       stg_nt<T>(rbW, O(6 + F_HZ) + bo, c.hz);
-      if (bulkrow && i >= ib + N && i < ie - N) return;
+      if (lean && sj < 0 && sjh < 0 && i >= ib + N && i < ie - N) return;   // no psi here
       const bool iin = i >= ib && i < ie, iin1 = i > ib && i < ie;
       const bool lkin = (lf & L3_KIN) != 0u, lkin1 = (lf & L3_KIN1) != 0u;
       int di = 0, ci = 0, dih = 0, cih = 0;
