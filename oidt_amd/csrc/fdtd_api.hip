@@ -602,10 +602,10 @@ constexpr size_t kCacheFields = (size_t)192 << 20;   // fields beyond this do no
 //
 // FP32 3D runs without monitors take the blocked step where their fields
 // exceed the last-level cache: the march is then bound by HBM.  March /
-// blocked, us per step: 4 guides of 128 x 96 x 320 (360 MiB) 271 / 249, 16 of
-// 64 x 48 x 193 (217) 254 / 177, 12 of 70 x 48 x 250 (230) 251 / 225, 16 of 110
-// x 70 x 400 985 / 626, 320 x 320 x 400 801 / 509; within the cache one 128 x
-// 96 x 320 (90) 61 / 86, 4 of 96 x 64 x 192..312 (141) 99 / 166.  In FP64 its
+// blocked, us per step: 4 guides of 128 x 96 x 320 (360 MiB) 270 / 242, 16 of
+// 64 x 48 x 193 (217) 252 / 171, 12 of 70 x 48 x 250 (230) 249 / 214, 16 of 110
+// x 70 x 400 978 / 592, 320 x 320 x 400 800 / 484; within the cache one 128 x
+// 96 x 320 (90) 60 / 84, 4 of 96 x 64 x 192..312 (141) 100 / 160.  In FP64 its
 // tiles own half the rows they step: 228 / 311 on those 4.
 //
 // The blocked steps give the two-kernel forms' bits in FP32, and at a chunk

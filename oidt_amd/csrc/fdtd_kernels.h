@@ -2552,15 +2552,16 @@ __global__ __launch_bounds__(kThreads, 4) void k_3d_halo(const Slot<T>* __restri
 // 16-wave block per CU: 4.5 us per plane and two steps, near enough the same
 // where every tile has a CU of its own).  Rows inside every update range, in
 // tiles without z slab, source or capture, take a body without selects inside
-// the x limits, with the x and y psi terms behind uniform branches.  The loads
-// run two positions ahead of their use.  For that the
-// compiler has to know how many are in flight, so the fields and y psi are
-// loaded without a branch around them, and the material comes as a dword (a
-// byte's zero extension waited for its load, and with it for all the others).
-// us per step, the march / this: 16 guides of 96 x 64 x 192..512 691 / 523
-// (560 before the loads ran ahead, 530 with the select-free body on the planes
-// and rows without psi only), 16 of 110 x 70 x 400 985 / 626, 320 x 320 x
-// 400 801 / 509, 128 x 96 x 320 61 / 86.
+// the x limits, with the x and y psi terms behind uniform branches.  Each
+// position waits once, at its start, for what the position before requested,
+// then stores the final plane and requests the next: the vector-memory counter
+// is in order, so a wait further down would also be for this position's own
+// requests and the stores before them.  (The material comes as a dword: a
+// byte's zero extension waited for its load, and with it for all the others.)
+// us per step, the march / this: 16 guides of 96 x 64 x 192..512 689 / 497
+// (560 with a position waiting for its own loads, 523 with counted waits that
+// stores came into), 16 of 110 x 70 x 400 978 / 592, 320 x 320 x 400 800 / 484,
+// 128 x 96 x 320 60 / 84.
 constexpr int kTb3Seg = 32;   // planes of a 3D blocked tile
 
 // One cell's state: fields, psi and material byte.
@@ -2758,15 +2759,14 @@ __global__ __launch_bounds__(64 * W) void k_3d_tb(const Slot<T>* __restrict__ sl
       const int sih = slab_h(i, ib, ie, N, dih, cih);
       const unsigned ix = ((unsigned)di * pl + jk) * es + (si == 1 ? xhi : 0u);
       const unsigned ixh = ((unsigned)dih * pl + jk) * es + (sih == 1 ? xhi : 0u);
-      // outside its slab a row or z lane reads element 0 (one line for the
-      // wave) and multiplies it by zero coefficients (z) or not at all (y)
-      const unsigned iy = sj >= 0 ? (((unsigned)i * N + dj) * nz + kc) * es : 0u;
-      const unsigned iyh = sjh >= 0 ? (((unsigned)i * N + djh) * nz + kc) * es : 0u;
+      // outside its slab a z lane reads element 0 (one line for the wave) and
+      // multiplies it by zero coefficients
+      const unsigned iy = (((unsigned)i * N + dj) * nz + kc) * es, iyh = (((unsigned)i * N + djh) * nz + kc) * es;
       const unsigned zrow = ((unsigned)i * ny + jc) * N * es;
       const unsigned iz = (lf & L3_SK) ? zrow + izk : 0u;
       const unsigned izh = (lf & L3_SKH) ? zrow + izkh : 0u;
       // (the zeros end the registers' life in a buffer that takes no new values)
-      c.qyx = c.qzx = c.ryx = c.rzx = c.qxz = c.qyz = c.rxz = c.ryz = T(0);
+      c.qyx = c.qzx = c.ryx = c.rzx = c.qxy = c.qzy = c.rxy = c.rzy = c.qxz = c.qyz = c.rxz = c.ryz = T(0);
       if (si >= 0) {
         c.qyx = ldg<T>(rbT, O(14) + ix);
         c.qzx = ldg<T>(rbT, O(15) + ix);
@@ -2781,10 +2781,14 @@ __global__ __launch_bounds__(64 * W) void k_3d_tb(const Slot<T>* __restrict__ sl
         c.rxz = ldg<T>(rbT, O(24) + izh);
         c.ryz = ldg<T>(rbT, O(25) + izh);
       }
-      c.qxy = ldg<T>(rbT, O(18) + iy);
-      c.qzy = ldg<T>(rbT, O(19) + iy);
-      c.rxy = ldg<T>(rbT, O(20) + iyh);
-      c.rzy = ldg<T>(rbT, O(21) + iyh);
+      if (sj >= 0) {
+        c.qxy = ldg<T>(rbT, O(18) + iy);
+        c.qzy = ldg<T>(rbT, O(19) + iy);
+      }
+      if (sjh >= 0) {
+        c.rxy = ldg<T>(rbT, O(20) + iyh);
+        c.rzy = ldg<T>(rbT, O(21) + iyh);
+      }
     };
 
     // One Yee step of cell c (plane i, step n0 + st): E, then H.  hyn, hzn:
@@ -3000,22 +3004,29 @@ __global__ __launch_bounds__(64 * W) void k_3d_tb(const Slot<T>* __restrict__ sl
     };
 
     // ---- the march.  At position p step 0 updates plane p - 2 and step 1
-    // plane p - 3, while plane p loads: each plane's cells load two positions
-    // before step 0 updates them (its Hy, Hz one position before, for step
-    // 0's update of the plane below).  Four cell buffers take the roles in
-    // turn (the loop is unrolled by four, so no buffer is copied, and no load
-    // in flight waits).
+    // plane p - 3, while plane p loads: each plane's fields load two positions
+    // before step 0 updates them (its Hy, Hz one position before, for step 0's
+    // update of the plane below), its psi one.  Four cell buffers take the
+    // roles in turn (the loop is unrolled by four, so no buffer is copied).
     T pey[TB], pez[TB];
 #pragma unroll
     for (int st = 0; st < TB; ++st) pey[st] = pez[st] = T(0);
+    const int pend = xo1 + TB;   // one position more stores the last plane
     auto position = [&](int p, Cell3<T>& ld, Cell3<T>& n1, Cell3<T>& c0, Cell3<T>& c1) {
       const unsigned lf = lflags = opaque_vgpr(lflags);
       ot = opaque_vgpr(ot);
-      // Loaded without a branch around it (planes past the last, and rows
-      // outside the grid, load the nearest one inside: no updated cell reads
-      // them, E rows end below ny - 1 and H rows start above row 0).
-      // The psi values follow one position later: they then live in three of
-      // the four buffers.
+      // What is in flight was requested a position ago.  Waiting for it here,
+      // once, leaves nothing to wait for in the rest of the position (the
+      // counter is in order: any later wait would also be for this position's
+      // requests, whose number the compiler does not know).
+      __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0)
+      // plane p - 4 is final, and its buffer takes plane p
+      if (p - 4 >= x0 && p - 4 < xo1 && (lf & L3_OWN)) store(ld, p - 4, lf);
+      if (p > pend) return;
+      // Planes past the last, and rows outside the grid, load the nearest one
+      // inside: no updated cell reads them, E rows end below ny - 1 and H rows
+      // start above row 0.  The psi values follow one position later: they then
+      // live in three of the four buffers.
       load_q(min(max(p - 1, xf), xl), lf, n1);
       load_f(min(p, xl), ld);
       // old Hx, Hz of both steps' planes for the wave below
@@ -3035,18 +3046,15 @@ __global__ __launch_bounds__(64 * W) void k_3d_tb(const Slot<T>* __restrict__ sl
         const T hzu = w + 1 < W ? xh[1][1][w + 1][lane] : c1.hz;
         step(c1, p - 3, 1, lf, c0.hy, c0.hz, hxu, hzu, pey[1], pez[1]);
       }
-      // plane p - 3 is final
-      if (p - 3 >= x0 && p - 3 < xo1 && (lf & L3_OWN)) store(c1, p - 3, lf);
     };
     lflags = opaque_vgpr(lflags);
     __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0): no load from before the march is waited for inside it
     Cell3<T> b0{}, b1{}, b2{}, b3{};
-    const int pend = xo1 + TB;
-    for (int p = xf; p <= pend; p += 4) {
+    for (int p = xf; p <= pend + 1; p += 4) {
       position(p, b0, b3, b2, b1);
-      if (p + 1 <= pend) position(p + 1, b1, b0, b3, b2);
-      if (p + 2 <= pend) position(p + 2, b2, b1, b0, b3);
-      if (p + 3 <= pend) position(p + 3, b3, b2, b1, b0);
+      if (p + 1 <= pend + 1) position(p + 1, b1, b0, b3, b2);
+      if (p + 2 <= pend + 1) position(p + 2, b2, b1, b0, b3);
+      if (p + 3 <= pend + 1) position(p + 3, b3, b2, b1, b0);
     }
     lds_barrier();   // the next tile reuses the exchange planes
   }
