@@ -309,9 +309,9 @@ int oidt_batch_remove(oidt_batch* b, int32_t slot);
  * picks the form itself: 2D batches whose monitors are single-point running
  * DFTs it can fold (lossy TMz: one per field, TEz: of Ey and Hz, TMz: none)
  * step in the blocked form, 8 steps per launch (FP32: the two-kernel form's
- * bits), and
- * oidt_batch_get_launch returns the defaults above, which a call with zeros
- * keeps.
+ * bits).  oidt_batch_get_launch then returns the form the resident runs step
+ * in (the defaults above while there is none), and a call that writes it back
+ * keeps that form.
  * No counterpart in the reference (fixed launch shapes, fdtd_main.py:263-273). */
 int oidt_batch_set_launch(oidt_batch* b, int32_t xchunk, int32_t grid_blocks, int32_t variant);
 

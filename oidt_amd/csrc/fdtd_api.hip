@@ -611,29 +611,29 @@ constexpr size_t kCacheFields = (size_t)192 << 20;   // fields beyond this do no
 // The blocked steps give the two-kernel forms' bits in FP32, and at a chunk
 // boundary every run's state is back in field set A, so a batch may change
 // between the two there (a run joins or leaves).
-void resolve_form(oidt_batch* b) {
-  b->run_variant = b->variant;
-  b->run_xchunk = b->xchunk;
-  if (b->auto_form && b->scheme != SCHEME_3D && blocked2d_monitors(b)) {
-    b->run_variant = 4;
-    b->run_xchunk = 8;
-  }
+struct Form { int variant, xchunk; };
+Form pick_form(const oidt_batch* b) {
+  Form f{b->variant, b->xchunk};
+  if (b->auto_form && b->scheme != SCHEME_3D && blocked2d_monitors(b)) f = {4, 8};
   if (b->auto_form && b->scheme == SCHEME_3D && b->precision == OIDT_F32 && !b->has_monitors() &&
-      field_bytes(b) > kCacheFields) {
-    b->run_variant = 4;
-    b->run_xchunk = 2;
-  }
+      field_bytes(b) > kCacheFields)
+    f = {4, 2};
   // The blocked steps address by 32-bit offsets: in 2D the high-side y psi from
   // the low-side array (three slabs in between), in 3D every array of a run
   // from its first field.  Runs beyond that take the two-kernel form.
-  if (b->run_variant == 4)
+  if (f.variant == 4)
     for (const auto& sh : b->slots)
       if (sh.used && (b->scheme == SCHEME_3D
                           ? sh.bytes > 4294967295ull
-                          : 3.0 * ((double)sh.desc.nx * sh.desc.num_cpml * (b->precision == OIDT_F64 ? 8 : 4) + 256.0) > 4294967295.0)) {
-        b->run_variant = b->scheme == SCHEME_3D ? 1 : 2;
-        b->run_xchunk = 4;
-      }
+                          : 3.0 * ((double)sh.desc.nx * sh.desc.num_cpml * (b->precision == OIDT_F64 ? 8 : 4) + 256.0) > 4294967295.0))
+        f = {b->scheme == SCHEME_3D ? 1 : 2, 4};
+  return f;
+}
+
+void resolve_form(oidt_batch* b) {
+  const Form f = pick_form(b);
+  b->run_variant = f.variant;
+  b->run_xchunk = f.xchunk;
   for (auto& sh : b->slots)
     if (sh.used && (b->chunks_enqueued - sh.admit_chunk) * kChunk < sh.desc.nt)
       sh.tb_run = run_tb(b->run_variant, b->run_xchunk);
@@ -1327,8 +1327,24 @@ int oidt_batch_add_indexed(oidt_batch* b, const oidt_run_desc* desc, const oidt_
 int oidt_batch_set_launch(oidt_batch* b, int32_t xchunk, int32_t grid_blocks, int32_t variant) {
   if (!b) return fail(OIDT_EINVAL, "null batch");
   if (variant < 0 || variant > 4) return fail(OIDT_EINVAL, "variant must be 0 (keep), 1, 2, 3 or 4");
+  if (grid_blocks < 0) return fail(OIDT_EINVAL, "negative grid size");
   if (variant == 0) variant = b->variant;
   const int xc = xchunk ? xchunk : b->xchunk;   // the depth this launch form will use
+  bool resident = false, started = false;
+  for (const auto& sh : b->slots) {
+    resident |= sh.used;
+    started |= sh.used && b->chunks_enqueued > sh.admit_chunk;
+  }
+  // The knobs oidt_batch_get_launch gave, written back where the checks below
+  // would refuse a caller's own choice of them: the library keeps choosing.
+  if (b->auto_form && resident && variant == 4) {
+    const Form f = pick_form(b);
+    if (f.variant == 4 && xc == f.xchunk && (started || b->has_monitors() || b->scheme == SCHEME_TMZ_LOSSY)) {
+      b->grid_override = grid_blocks;
+      b->dirty = true;
+      return OIDT_OK;
+    }
+  }
   if (variant == 4) {
     if (b->scheme == SCHEME_3D) {
       if (xc != 2) return fail(OIDT_EINVAL, "the blocked 3D step takes 2 steps per launch");
@@ -1347,7 +1363,6 @@ int oidt_batch_set_launch(oidt_batch* b, int32_t xchunk, int32_t grid_blocks, in
   const bool fused_only = xc == 12 || xc == 20 || xc == 24;
   if (!pow2 && !(fused_only && variant == 3))
     return fail(OIDT_EINVAL, "xchunk must be 0 (keep), 1, 2, 4, 8, 16 or 32 (also 12, 20 or 24 for the fused step)");
-  if (grid_blocks < 0) return fail(OIDT_EINVAL, "negative grid size");
   if (variant == 3 && b->scheme == SCHEME_TMZ_LOSSY)
     return fail(OIDT_EINVAL, "the lossy TMz form has no fused step (variant 1 or 2)");
   if (variant >= 3 && b->has_monitors())
@@ -1364,9 +1379,13 @@ int oidt_batch_set_launch(oidt_batch* b, int32_t xchunk, int32_t grid_blocks, in
 
 int oidt_batch_get_launch(const oidt_batch* b, int32_t* xchunk, int32_t* grid_blocks, int32_t* variant) {
   if (!b) return fail(OIDT_EINVAL, "null batch");
-  if (xchunk) *xchunk = b->xchunk;
+  // the form the resident runs step in, where the library picks it
+  Form f{b->variant, b->xchunk};
+  for (const auto& sh : b->slots)
+    if (sh.used && b->auto_form) f = pick_form(b);
+  if (xchunk) *xchunk = f.xchunk;
   if (grid_blocks) *grid_blocks = b->grid_override;
-  if (variant) *variant = b->variant;
+  if (variant) *variant = f.variant;
   return OIDT_OK;
 }
 
