@@ -308,8 +308,9 @@ int oidt_batch_remove(oidt_batch* b, int32_t slot);
  * nor the blocked step's depth (OIDT_ESTATE).  Until the first call the library
  * picks the form itself: 2D batches whose monitors are single-point running
  * DFTs it can fold (lossy TMz: one per field, TEz: of Ey and Hz, TMz: none)
- * step in the blocked form, 8 steps per launch (FP32: the two-kernel form's
- * bits).  oidt_batch_get_launch then returns the form the resident runs step
+ * step in the blocked form, 8 steps per launch, FP32 3D batches without
+ * monitors whose fields exceed 192 MiB and whose runs the tiles cover well in
+ * the blocked 3D form (FP32: the two-kernel forms' bits).  oidt_batch_get_launch then returns the form the resident runs step
  * in (the defaults above while there is none), and a call that writes it back
  * keeps that form.
  * No counterpart in the reference (fixed launch shapes, fdtd_main.py:263-273). */

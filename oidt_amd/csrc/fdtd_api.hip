@@ -591,6 +591,33 @@ size_t field_bytes(const oidt_batch* b) {
 }
 constexpr size_t kCacheFields = (size_t)192 << 20;   // fields beyond this do not stay in the 256 MiB last-level cache
 
+// Lane-cells the blocked 3D step takes through its positions per cell of the
+// batch, tiles of 32 planes x 12 rows x 60 z-cells on the CUs in rounds of one
+// tile each: 1.6 where the tiles fit, 4.5 for many small runs just past the
+// tile edges.  It costs 3.5..5 us per position and CU however many of these it
+// owns, the march 17..38 ps per cell.  Blocked / march time over 38 batches of
+// 188..1318 MiB: 0.50..1.01 below 3 (20 of 97 x 61 x 130: 379 / 376 us per
+// step), 0.80..1.07 from there to 3.3 (40 of 66 x 50 x 80 308 / 386, 27 of 65 x
+// 49 x 121 295 / 275), 1.13 and 0.95 at 3.31 and 3.68 (30 of 65 x 61 x 121 378 /
+// 335, 30 of 129 x 37 x 121 486 / 510), 1.02..1.28 above 4 (110 of 33 x 37 x 61
+// 348 / 271, 93 of 40 x 37 x 61 350 / 319, 220 of 65 x 37 x 61 1245 / 1185).
+constexpr double kCover3d = 3.3;
+double blocked3d_cover(const oidt_batch* b) {
+  const int tb = 2, waves = tb3_waves(b->precision), ty = waves - 2 * tb, tz = kBX - 2 * tb, cus = 256;
+  double tiles = 0, positions = 0, cells = 0;
+  for (const auto& sh : b->slots) {
+    if (!sh.used) continue;
+    const oidt_run_desc& d = sh.desc;
+    const double across = (double)((d.ny + ty - 1) / ty) * ((d.nz + tz - 1) / tz);
+    for (int x0 = 0; x0 < d.nx; x0 += kTb3Seg) {
+      tiles += across;
+      positions += across * (std::min(x0 + kTb3Seg, d.nx) + tb - std::max(x0 - tb, 0) + 1);
+    }
+    cells += (double)d.nx * d.ny * d.nz;
+  }
+  return cells > 0 ? positions * (std::ceil(tiles / cus) * cus / tiles) * waves * kBX / cells : 0;
+}
+
 // The form the launches use where the caller has not set the launch knobs (to
 // keep them counts as setting them).
 //
@@ -601,12 +628,13 @@ constexpr size_t kCacheFields = (size_t)192 << 20;   // fields beyond this do no
 // 800..4000 x 240 353 / 57.
 //
 // FP32 3D runs without monitors take the blocked step where their fields
-// exceed the last-level cache: the march is then bound by HBM.  March /
-// blocked, us per step: 4 guides of 128 x 96 x 320 (360 MiB) 270 / 242, 16 of
-// 64 x 48 x 193 (217) 252 / 171, 12 of 70 x 48 x 250 (230) 249 / 214, 16 of 110
-// x 70 x 400 978 / 592, 320 x 320 x 400 800 / 484; within the cache one 128 x
-// 96 x 320 (90) 60 / 84, 4 of 96 x 64 x 192..312 (141) 100 / 160.  In FP64 its
-// tiles own half the rows they step: 228 / 311 on those 4.
+// exceed the last-level cache (the march is then bound by HBM) and its tiles
+// cover the runs (blocked3d_cover).  March / blocked, us per step: 4 guides of
+// 128 x 96 x 320 (360 MiB) 267 / 242, 16 of 64 x 48 x 193 (217) 255 / 171, 12
+// of 70 x 48 x 250 (231) 251 / 214, 16 of 110 x 70 x 400 992 / 593, 320 x 320 x
+// 400 800 / 486; within the cache one 128 x 96 x 320 (90) 60 / 84, 4 of 96 x 64
+// x 192..312 (141) 100 / 160.  In FP64 its tiles own half the rows they step:
+// 228 / 311 on those 4.
 //
 // The blocked steps give the two-kernel forms' bits in FP32, and at a chunk
 // boundary every run's state is back in field set A, so a batch may change
@@ -616,7 +644,7 @@ Form pick_form(const oidt_batch* b) {
   Form f{b->variant, b->xchunk};
   if (b->auto_form && b->scheme != SCHEME_3D && blocked2d_monitors(b)) f = {4, 8};
   if (b->auto_form && b->scheme == SCHEME_3D && b->precision == OIDT_F32 && !b->has_monitors() &&
-      field_bytes(b) > kCacheFields)
+      field_bytes(b) > kCacheFields && blocked3d_cover(b) <= kCover3d)
     f = {4, 2};
   // The blocked steps address by 32-bit offsets: in 2D the high-side y psi from
   // the low-side array (three slabs in between), in 3D every array of a run

@@ -7,6 +7,7 @@ from oidt_amd import variants
 from oidt_amd.solver import Batch, Monitor
 
 from test_gpu_blocked2d import outcome, run, same, small
+from test_gpu_blocked3d import strip
 
 LOSSY = dict(sgl_wg_length=1.5e-6, port_length=0.3e-6, points_per_wl=16, ny_clad_wl=0.4, buffer_xhat=5, num_cpml=6)
 
@@ -72,4 +73,18 @@ def test_reported_form_of_lossy_runs():
     b.advance(1)
     write_back(b)
     assert b.launch() == (4, 8, 0)
+    b.close()
+
+
+@pytest.mark.gpu
+# fields of 205 and 231 MiB
+@pytest.mark.parametrize('copies,nx,ny,nz,form', [(120, 33, 37, 61, (1, 4, 0)), (12, 70, 48, 250, (4, 2, 0))])
+def test_large_3d_batches_take_the_blocked_form_where_its_tiles_cover(copies, nx, ny, nz, form):
+    """Runs just past the tile edges stay with the march."""
+    a = strip(nx, ny, nz, 64)
+    print('case', copies, nx, ny, nz, flush=True)
+    b = Batch('3d', np.float32, max_slots=copies)
+    for _ in range(copies):
+        b.add(*a)
+    assert b.launch() == form
     b.close()
