@@ -93,6 +93,7 @@ struct MonHost {
   void* im = nullptr;
   double* cs = nullptr;
   size_t cells = 0;
+  bool finite = true;   // its weights
 };
 
 struct SlotHost {
@@ -566,7 +567,8 @@ int tb3_waves(int precision) { return precision == OIDT_F64 ? 8 : 16; }
 
 // Whether the blocked 2D step can fold the batch's monitors: single-point
 // running DFTs, at most one per field of a run (TEz: of Ey and Hz), as the
-// scattering-loss drivers attach them.
+// scattering-loss drivers attach them.  (Their weights are finite: the blocked
+// step leaves out the cells that stay zero.)
 bool blocked2d_monitors(const oidt_batch* b) {
   for (const auto& sh : b->slots) {
     if (!sh.used) continue;
@@ -574,7 +576,7 @@ bool blocked2d_monitors(const oidt_batch* b) {
     for (const MonHost& mh : sh.mons) {
       const oidt_monitor_desc& d = mh.d;
       const unsigned bit = 1u << d.field;
-      if (d.mode != OIDT_MON_DFT || d.npts != 1 || d.off[0][0] || d.off[0][1] || d.off[0][2] || (seen & bit)) return false;
+      if (d.mode != OIDT_MON_DFT || !mh.finite || d.npts != 1 || d.off[0][0] || d.off[0][1] || d.off[0][2] || (seen & bit)) return false;
       if (b->scheme == SCHEME_TMZ || (b->scheme == SCHEME_TEZ && d.field == F_EX)) return false;
       seen |= bit;
     }
@@ -1714,6 +1716,8 @@ int oidt_batch_add_monitor(oidt_batch* b, int32_t slot, const oidt_monitor_desc*
   mh.d = *m;
   mh.d.cs = nullptr;
   mh.cells = cells;
+  if (m->mode == OIDT_MON_DFT)
+    for (int64_t k = 0; k < 2 * (int64_t)m->nrec; ++k) mh.finite = mh.finite && std::isfinite(m->cs[k]);
   const size_t rbytes = (m->mode == OIDT_MON_DFT ? cells : cells * (size_t)m->nrec) * esz;
   auto undo = [&]() {
     for (void* p : {mh.re, mh.im, static_cast<void*>(mh.cs)})

@@ -288,23 +288,25 @@ __device__ __forceinline__ void blocked_step_2d(const Slot<T>* __restrict__ slot
           if ((f & 16) && yxh) qx[q] = ldg<T>(psiA[psi_id(R::QX, 0, rh >= kHi)], (unsigned)((rh & (kHi - 1)) * ny + jc) * es);
         }
       }
-      // A cell outside a component's update range keeps its value by a zero
-      // factor (its coefficient, 1/kappa or db), so the steps need no range
-      // selects (only a non-finite neighbour could change it).  dbr: db of the
-      // rows of TMz Hy / TEz Hz.
-      T dbr = db, dtr = dtmu;   // dtr: dt / mu of the lossy form's Hy psi
-      if (CLS != 1) {
-        dbr = yxh ? db : T(0);
-        dtr = yxh ? dtr : T(0);
-#pragma unroll
-        for (int q = 0; q < K; ++q) {
-          const int f = kX ? at(lf, q) : 3;
-          const bool x0 = (f & 1) != 0, x1 = (f & 2) != 0;
-          cb0[q] = (tm ? x0 : x1) && yin ? cb0[q] : T(0);
-          if (!tm) cb1[q] = x0 && yin1 ? cb1[q] : T(0);
-          if (lossy) cb1[q] = x0 && yin ? cb1[q] : T(1);
-        }
-      }
+      // A cell outside a component's update range keeps its value by a select in
+      // every step where an updated neighbour along x or y reads it (TMz A / C,
+      // TEz A / A, lossy TMz B / B) and on the source planes (TMz B, TEz A: the
+      // source drives cells outside the ranges too).  The other cells outside a
+      // range hold zero and are read by nothing that is updated: the steps let
+      // them go, captures and the final store take the zero, and monitors fold
+      // nothing there.  (A zero factor instead of the selects also keeps a
+      // finite cell, but turns it NaN beside an infinite neighbour.  A 600 x 240
+      // FP64 solve, the case with the largest difference: 8.44 ms with zero
+      // factors, 8.54 so.)
+      constexpr bool sxA = !lossy, syA = !tm;
+      constexpr bool sxB = lossy, syB = lossy;
+      constexpr bool sxC = false, syC = tm && !lossy;
+      // update planes (bits of the x flags) and rows
+      constexpr unsigned upA = 2u, upB = 1u, upC = tm && !lossy ? 1u : 2u;
+      const bool yA = yxh, yB = yxe, yC = tm ? yin1 : yin;
+      auto updates = [&](bool sx, unsigned xin, bool sy, bool yr) {
+        return (!kX || !sx || xin != 0u) && (CLS == 1 || !sy || yr);
+      };
       // With few planes the flags, masks and slab coefficients stay in scalar
       // registers over the steps; with many they are formed again in every
       // step (they would spill).
@@ -324,7 +326,7 @@ __device__ __forceinline__ void blocked_step_2d(const Slot<T>* __restrict__ slot
           const T dy = lane_prev(c[q]) - c[q];
           const T ch = cb0[q];
           T e = fmadd(cb1[q], bf[q], ch * fmadd(dy, ikye, dx * kx[q]));
-          if (kSp && (f & 4u)) e = jsrc ? e - jv : e;
+          if (kSp && (f & 4u)) e = jsrc ? e - jv : e;   // (the box lies inside the update range)
           if (CLS != 1) {
             const T chdx = ch * dxT;
             if (kX && (f & 8u)) {
@@ -334,11 +336,12 @@ __device__ __forceinline__ void blocked_step_2d(const Slot<T>* __restrict__ slot
             py[q] = fmadd(cey, dy, bey * py[q]);
             e = sye >= 0 ? fmadd(chdx, py[q], e) : e;
           }
-          bf[q] = e;
+          bf[q] = updates(sxB, f & upB, syB, yB) ? e : bf[q];
         } else if constexpr (tm) {
           const T dy = lane_next(c[q]) - c[q];
           const T cb = cb0[q];
           T e = fmadd(cb, fmadd(dx, kx[q], -(dy * ikye)), bf[q]);
+          const T kept = kSp && jsrc ? bf[q] - jv : bf[q];
           if (kSp && (f & 4u)) e = jsrc ? e - jv : e;
           if (kX && (f & 8u)) {
             px[q] = fmadd(coef(lbe, q), px[q], coef(lce, q) * dx);
@@ -348,6 +351,7 @@ __device__ __forceinline__ void blocked_step_2d(const Slot<T>* __restrict__ slot
             psi_step(py[q], bey, cey * dy);
             e = sye >= 0 ? fmadd(-cb, py[q], e) : e;
           }
+          if (kSp && (f & 4u)) e = (f & upB) && yB ? e : kept;
           bf[q] = e;
         } else {
           const T dy = lane_next(a[q]) - a[q];
@@ -365,8 +369,9 @@ __device__ __forceinline__ void blocked_step_2d(const Slot<T>* __restrict__ slot
           bf[q] = ey;
         }
         if (kSp && (f & 96u) && jcap) {
-          if (f & 32u) cap(t, 0, bf[q]);
-          if (f & 64u) cap(t, 3, bf[q]);
+          const T v = sxB || (tm && (f & 4u)) || ((f & upB) && yB) ? bf[q] : T(0);
+          if (f & 32u) cap(t, 0, v);
+          if (f & 64u) cap(t, 3, v);
         }
       };
       // H half-step of plane q; dn: B of plane q - 1 (lossy: q + 1)
@@ -377,16 +382,17 @@ __device__ __forceinline__ void blocked_step_2d(const Slot<T>* __restrict__ slot
         if constexpr (lossy) {
           const T dy = bf[q] - lane_next(bf[q]);
           T hx = fmadd(db * dy, ikyh, c[q]);
-          h = fmadd((CLS != 1 ? dbr : db) * dx, kh[q], a[q]);
+          h = fmadd(db * dx, kh[q], a[q]);
           if (CLS != 1) {
             if (kX && (f & 16u)) {
               qx[q] = fmadd(coef(lch, q), dx, coef(lbh, q) * qx[q]);
-              h = fmadd(dtr, qx[q], h);
+              h = fmadd(dtmu, qx[q], h);
             }
             qy[q] = fmadd(chy, dy, bhy * qy[q]);
             hx = syh >= 0 ? fmadd(dtmu, qy[q], hx) : hx;
           }
-          if (!kX || (f & 2u)) c[q] = hx;
+          c[q] = updates(sxC, f & upC, syC, yC) ? hx : c[q];
+          h = updates(sxA, f & upA, syA, yA) ? h : a[q];
         } else if constexpr (tm) {
           const T dy = bf[q] - lane_prev(bf[q]);
           T hx = fmadd(db * -dy, ikyh, c[q]);
@@ -394,33 +400,40 @@ __device__ __forceinline__ void blocked_step_2d(const Slot<T>* __restrict__ slot
             psi_step(qy[q], bhy, chy * dy);
             hx = syh >= 0 ? fmadd(-db, qy[q], hx) : hx;
           }
-          if (!kX || (f & 1u)) c[q] = hx;
-          h = fmadd((CLS != 1 ? dbr : db) * dx, kh[q], a[q]);
-          if (kX && (f & 16u)) {
-            qx[q] = fmadd(coef(lbh, q), qx[q], coef(lch, q) * dx);
-            h = fmadd(dbr, qx[q], h);
+          c[q] = updates(sxC, f & upC, syC, yC) ? hx : c[q];
+          h = a[q];
+          if (!kX || (f & upA)) {
+            h = fmadd(db * dx, kh[q], h);
+            if (kX && (f & 16u)) {
+              qx[q] = fmadd(coef(lbh, q), qx[q], coef(lch, q) * dx);
+              h = fmadd(db, qx[q], h);
+            }
           }
         } else {
           const T dy = c[q] - lane_prev(c[q]);
-          const T d = CLS == 1 ? db : dbr;
-          h = fmadd(d, fmadd(dy, ikyh, -(dx * kh[q])), a[q]);
-          if (kX && !(f & 2u)) h = a[q];
-          if (kSp && (f & 4u)) h = jsrc ? h - jv : h;
+          T kept = a[q];
+          h = fmadd(db, fmadd(dy, ikyh, -(dx * kh[q])), a[q]);
+          if (kSp && (f & 4u)) {
+            h = jsrc ? h - jv : h;
+            kept = jsrc ? kept - jv : kept;
+          }
           if (kX && (f & 16u)) {
             qx[q] = fmadd(coef(lbh, q), qx[q], coef(lch, q) * dx);
-            h = fmadd(-d, qx[q], h);
+            h = fmadd(-db, qx[q], h);
           }
           if (CLS != 1) {
             psi_step(qy[q], bhy, chy * dy);
-            h = syh >= 0 && (!kX || (f & 2u)) ? fmadd(d, qy[q], h) : h;
+            h = syh >= 0 ? fmadd(db, qy[q], h) : h;
           }
+          h = updates(sxA, f & upA, syA, yA) ? h : kept;
         }
         a[q] = h;
         if (kSp && (f & 480u) && jcap) {
-          if (f & 32u) cap(t, 1, h);
-          if (f & 128u) cap(t, 2, h);
-          if (f & 64u) cap(t, 4, h);
-          if (f & 256u) cap(t, 5, h);
+          const T v = syA || yA ? h : T(0);   // its planes are selected
+          if (f & 32u) cap(t, 1, v);
+          if (f & 128u) cap(t, 2, v);
+          if (f & 64u) cap(t, 4, v);
+          if (f & 256u) cap(t, 5, v);
         }
       };
       // ---- monitors: running sums of this wave's cells, weights (lane t:
@@ -431,6 +444,19 @@ __device__ __forceinline__ void blocked_step_2d(const Slot<T>* __restrict__ slot
       unsigned mvalid[NM];
       const Monitor<T>* mon[NM];
       bool mafter[NM];
+      // the own rows and planes [lo, hi) of monitor m of role r: of its box, and
+      // inside the update range unless the steps keep the role's other cells
+      struct MonBox { int lo, hi; bool row; };
+      auto box = [&](int r, const Monitor<T>& m) {
+        MonBox x;
+        const int xb = r == 0 ? (sxA ? 0 : lossy ? 0 : ib + 1) : r == 1 ? (sxB ? 0 : ib) : (lossy ? 0 : ib + 1);
+        const int xe = (r == 0 ? sxA : r == 1 ? sxB : sxC) ? nx : ie;
+        x.lo = max(max(i0, m.x0), xb);
+        x.hi = min(min(i0 + TX, m.x0 + m.ex), xe);
+        x.row = lane >= TB && lane < TB + TY && j >= m.y0 && j < m.y0 + m.ey &&
+                (r == 0 ? syA || yA : r == 1 ? syB || yB : syC || yC);
+        return x;
+      };
       if constexpr (MON != 0) {
         const int2 sm = smon[tl.x];
 #pragma unroll
@@ -452,11 +478,11 @@ __device__ __forceinline__ void blocked_step_2d(const Slot<T>* __restrict__ slot
             lci[r] = has ? m.cs[2 * rec + 1] : 0.0;
             msc[r] = m.scale;
             mafter[r] = m.after_h != 0;
+            const MonBox x = box(r, m);
 #pragma unroll
             for (int q = 0; q < K; ++q) {
               const int i = ib0 + q, cell = (i - m.x0) * m.ey + (j - m.y0);
-              const bool in = i >= i0 && i < i0 + TX && i >= m.x0 && i < m.x0 + m.ex && lane >= TB && lane < TB + TY &&
-                              j >= m.y0 && j < m.y0 + m.ey;
+              const bool in = i >= x.lo && i < x.hi && x.row;
               mre[r][q] = in ? m.re[cell] : T(0);
               mim[r][q] = in ? m.im[cell] : T(0);
             }
@@ -511,11 +537,12 @@ __device__ __forceinline__ void blocked_step_2d(const Slot<T>* __restrict__ slot
         for (int r = 0; r < NM; ++r) {
           if (!(MON & (1 << r)) || !mvalid[r]) continue;
           const Monitor<T>& m = *mon[r];
+          const MonBox x = box(r, m);
+          if (!x.row) continue;
 #pragma unroll
           for (int q = 0; q < K; ++q) {
             const int i = ib0 + q, cell = (i - m.x0) * m.ey + (j - m.y0);
-            if (i >= i0 && i < i0 + TX && i >= m.x0 && i < m.x0 + m.ex && lane >= TB && lane < TB + TY && j >= m.y0 &&
-                j < m.y0 + m.ey) {
+            if (i >= x.lo && i < x.hi) {
               m.re[cell] = mre[r][q];
               m.im[cell] = mim[r][q];
             }
@@ -551,10 +578,14 @@ __device__ __forceinline__ void blocked_step_2d(const Slot<T>* __restrict__ slot
         for (int q = 0; q < K; ++q) {
           const int i = ib1 + q;
           if (i < i0 || i >= i0 + TX || i >= nx) continue;
+          // selected in every step, or updated
+          auto clean = [&](bool sx, unsigned up, bool sy, bool yr) {
+            return (!kX || sx || ((unsigned)xf[q] & up) != 0u) && (CLS == 1 || sy || yr);
+          };
           const unsigned idx = (unsigned)i * ny + js;
-          stg_nt<T>(oA, idx * es, a[q]);
-          stg_nt<T>(oB, idx * es, bf[q]);
-          stg_nt<T>(oC, idx * es, c[q]);
+          stg_nt<T>(oA, idx * es, clean(sxA, upA, syA, yxhs) ? a[q] : T(0));
+          stg_nt<T>(oB, idx * es, clean(sxB, upB, syB, yxes) || (kSp && tm && (xf[q] & 4)) ? bf[q] : T(0));
+          stg_nt<T>(oC, idx * es, clean(sxC, upC, syC, tm ? yins1 : yins) ? c[q] : T(0));
         }
         if (CLS != 1 && !yplain) {
           int dyes = 0, dyhs = 0, unused = 0;
