@@ -2759,8 +2759,8 @@ __global__ __launch_bounds__(64 * W) void k_3d_tb(const Slot<T>* __restrict__ sl
       const int sih = slab_h(i, ib, ie, N, dih, cih);
       const unsigned ix = ((unsigned)di * pl + jk) * es + (si == 1 ? xhi : 0u);
       const unsigned ixh = ((unsigned)dih * pl + jk) * es + (sih == 1 ? xhi : 0u);
-      // outside its slab a z lane reads element 0 (one line for the wave) and
-      // multiplies it by zero coefficients
+      // outside its slab a z lane reads element 0 (one line for the wave), and
+      // its update leaves the value out
       const unsigned iy = (((unsigned)i * N + dj) * nz + kc) * es, iyh = (((unsigned)i * N + djh) * nz + kc) * es;
       const unsigned zrow = ((unsigned)i * ny + jc) * N * es;
       const unsigned iz = (lf & L3_SK) ? zrow + izk : 0u;
@@ -2847,7 +2847,7 @@ __global__ __launch_bounds__(64 * W) void k_3d_tb(const Slot<T>* __restrict__ sl
         const T dHy = hyk - c.hy;
         T v = fmadd(cb, fmadd(dHz, iky, -(dHy * ikz)), vx);
         if (sj >= 0) { const T qv = fmadd(cej, dHz, bej * c.qxy); c.qxy = qv; v = fmadd(cb, qv, v); }
-        if (zs) { const T qv = fmadd(cek, dHy, bek * c.qxz); c.qxz = qv; v = fmadd(-cb, qv, v); }
+        if (zs) { const T qv = fmadd(cek, dHy, bek * c.qxz); c.qxz = qv; v = (lf & L3_SK) ? fmadd(-cb, qv, v) : v; }
         vx = lkin ? v : vx;
       }
       const bool srcp = srcx && (lf & L3_SRCE) != 0u;
@@ -2858,7 +2858,7 @@ __global__ __launch_bounds__(64 * W) void k_3d_tb(const Slot<T>* __restrict__ sl
         T v = fmadd(cb, fmadd(dHx, ikz, -(dHz * ikx)), vy);
         v = srcp ? v - jv : v;
         if (si) { const T qv = fmadd(xc[0][u], c.qyx, xc[1][u] * dHz); c.qyx = qv; v = fmadd(-cb, qv, v); }
-        if (zs) { const T qv = fmadd(cek, dHx, bek * c.qyz); c.qyz = qv; v = fmadd(cb, qv, v); }
+        if (zs) { const T qv = fmadd(cek, dHx, bek * c.qyz); c.qyz = qv; v = (lf & L3_SK) ? fmadd(cb, qv, v) : v; }
         vy = lkin ? v : (srcp ? vy - jv : vy);
       } else {
         vy = srcp ? vy - jv : vy;
@@ -2919,7 +2919,7 @@ __global__ __launch_bounds__(64 * W) void k_3d_tb(const Slot<T>* __restrict__ sl
         const T dEz = vz - ezm;
         T v = fmadd(db, fmadd(dEy, ikzh, -(dEz * ikyh)), hx);
         if (sjh >= 0) { const T qv = fmadd(bhj, c.rxy, chj * dEz); c.rxy = qv; v = fmadd(-db, qv, v); }
-        if (zs) { const T qv = fmadd(bhk, c.rxz, chk * dEy); c.rxz = qv; v = fmadd(db, qv, v); }
+        if (zs) { const T qv = fmadd(bhk, c.rxz, chk * dEy); c.rxz = qv; v = (lf & L3_SKH) ? fmadd(db, qv, v) : v; }
         hx = lkin1 ? v : hx;
       }
       const bool srch = srcx && (lf & L3_SRCH) != 0u;
@@ -2929,7 +2929,7 @@ __global__ __launch_bounds__(64 * W) void k_3d_tb(const Slot<T>* __restrict__ sl
         const T dEx = vx - exk;
         T v = fmadd(db, fmadd(dEz, ikxh, -(dEx * ikzh)), hy);
         if (sih) { const T qv = fmadd(xc[2][u], c.ryx, xc[3][u] * dEz); c.ryx = qv; v = fmadd(db, qv, v); }
-        if (zs) { const T qv = fmadd(bhk, c.ryz, chk * dEx); c.ryz = qv; v = fmadd(-db, qv, v); }
+        if (zs) { const T qv = fmadd(bhk, c.ryz, chk * dEx); c.ryz = qv; v = (lf & L3_SKH) ? fmadd(-db, qv, v) : v; }
         hy = lkin1 ? v : hy;
       }
       if (iin1 && jin1) {

@@ -10,6 +10,7 @@ from oidt_amd import variants
 from oidt_amd.solver import Batch, Monitor, Solver
 
 from test_gpu_blocked2d import FIELDS, run, small
+from test_gpu_blocked3d import alone, strip
 
 
 def infinite(s, step=2):
@@ -93,4 +94,15 @@ def test_infinite_weights_take_the_monitor_kernel():
         b.close()
     assert np.isnan(out[0][0][:, 0]).all()      # the first row stays zero
     for x, y in zip(*out):
+        assert np.array_equal(x, y, equal_nan=True)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('nx,ny,nz,direction', [(33, 37, 61, 'f'), (64, 48, 120, 'b'), (65, 49, 121, 'f')])
+def test_blocked_3d_keeps_the_marchs_cells(nx, ny, nz, direction):
+    s, fg = strip(nx, ny, nz, 45)
+    print('case', nx, ny, nz, direction, flush=True)
+    got, ref = (alone((infinite(s), fg), launch, direction) for launch in ((2, 0, 4), (4, 0, 1)))
+    assert any(not np.isfinite(x).all() for x in ref)
+    for x, y in zip(got, ref):
         assert np.array_equal(x, y, equal_nan=True)
