@@ -151,11 +151,21 @@ def _window_cells(s):
     return (wy[1] - wy[0]) * ((wx[1] - wx[0]) if wx else 1)
 
 
+def _given(arrays):
+    """(inputs, material) as the library is given them: the material index of a
+    ``RunArrays`` whose ``inputs`` and CB maps are its own, else None and what
+    ``inputs()`` returns."""
+    own = (isinstance(arrays, RunArrays) and getattr(arrays.inputs, '__func__', None) is RunArrays.inputs
+           and type(arrays).cb is RunArrays.cb)
+    if own and arrays.material is not None:
+        return arrays.inputs_without_maps(), arrays.material
+    return arrays.inputs(), None
+
+
 def _create(arrays, desc):
     """(handle, inputs) of a single run."""
     h = C.c_void_p()
-    material = getattr(arrays, 'material', None)
-    r = arrays.inputs() if material is None else arrays.inputs_without_maps()
+    r, material = _given(arrays)
     if material is None:
         check(lib().oidt_solver_create(C.byref(desc), C.byref(r), C.byref(h)))
     else:
@@ -290,8 +300,7 @@ class Batch:
         describes it to the Python side (nt, precision, shape, frequencies)."""
         d = arrays.desc()
         slot = C.c_int32()
-        material = getattr(arrays, 'material', None)
-        r = arrays.inputs() if material is None else arrays.inputs_without_maps()
+        r, material = _given(arrays)
         if material is None:
             check(lib().oidt_batch_add(self.h, C.byref(d), C.byref(r), C.byref(slot)))
         else:
