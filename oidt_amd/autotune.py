@@ -5,7 +5,8 @@ candidate (kernel form, x-chunk depth, grid cap) on a copy of the real batch
 by replaying its chunk graph, re-times the two fastest over more chunks, and
 keeps the one with the smallest time per step.  The copies last long enough
 that every timed launch does a whole step for every run.  Results are cached
-per workload class in a JSON file so a serving process tunes each class once.
+per workload class in a JSON file so a serving process tunes each class once;
+a choice measured with another build of the library is measured again.
 
 Kernel forms: 1 = per-plane march, 2 = batched loads (two launches per step),
 3 = fused Yee step (one launch per step), 4 = temporally blocked step
@@ -13,6 +14,7 @@ Kernel forms: 1 = per-plane march, 2 = batched loads (two launches per step),
 planes each thread or wave owns along x.
 """
 import dataclasses
+import hashlib
 import json
 import os
 import time
@@ -42,6 +44,12 @@ def workload_class(setups):
     cells = sum(s.cells for s in setups)
     return '%s-%s-n%d-c%d' % (s0.scheme, np.dtype(s0.precision).name, len(setups),
                               int(round(np.log2(max(cells, 1)))))
+
+
+def build_id():
+    """Identifies the library file whose kernels a choice was measured with."""
+    with open(_lib.LIB_PATH, 'rb') as fh:
+        return hashlib.sha256(fh.read()).hexdigest()[:16]
 
 
 # chunks replayed per candidate: a warm-up chunk, then TIMED_CHUNKS (first
@@ -91,13 +99,14 @@ def tune(runs, candidates=None, cache_path=DEFAULT_CACHE, use_cache=True, verbos
     setups = [s for s, _ in runs]
     key = workload_class(setups)
     cache = {}
+    build = build_id() if cache_path else None
     if use_cache and cache_path and os.path.exists(cache_path):
         try:
             with open(cache_path) as fh:
                 cache = json.load(fh)
         except (OSError, ValueError):
             cache = {}
-        if key in cache:
+        if key in cache and cache[key].get('build') == build:
             return tuple(cache[key]['choice']), cache[key]['times']
     scheme = setups[0].scheme
     cands = candidates or CANDIDATES[scheme]
@@ -118,7 +127,7 @@ def tune(runs, candidates=None, cache_path=DEFAULT_CACHE, use_cache=True, verbos
     best = min(top, key=times.get)
     choice = tuple(int(v) for v in best.split(','))
     if cache_path:
-        cache[key] = {'choice': list(choice), 'times': times}
+        cache[key] = {'choice': list(choice), 'times': times, 'build': build}
         os.makedirs(os.path.dirname(cache_path), exist_ok=True)
         with open(cache_path, 'w') as fh:
             json.dump(cache, fh, indent=1, sort_keys=True)
