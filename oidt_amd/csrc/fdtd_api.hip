@@ -1532,7 +1532,13 @@ int oidt_batch_read_dft_plane(oidt_batch* b, int32_t slot, int32_t port, int32_t
     for (size_t e = at / 16, end = (at + n) / 16; e < end;) {
       const size_t row = e / len, c = e - row * len, m = std::min(len - c, end - e);
       const size_t f = row / rows, x = x0 + row % rows;
-      std::memcpy(out + 2 * ((f * xs + x) * d.ny + N + c), p, m * 16);
+      // re + 1j * im as complex arithmetic forms it (a zero's sign, non-finite parts)
+      double* o = out + 2 * ((f * xs + x) * d.ny + N + c);
+      const double* v = reinterpret_cast<const double*>(p);
+      for (size_t k = 0; k < m; ++k) {
+        o[2 * k] = v[2 * k] + 0.0 * v[2 * k + 1];
+        o[2 * k + 1] = 0.0 + v[2 * k + 1];
+      }
       p += m * 16;
       e += m;
     }

@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 
 from oidt_amd import variants
-from oidt_amd.solver import Batch, Monitor, Solver
+from oidt_amd.solver import COMP_KEYS, Batch, Monitor, Solver
 
 from test_gpu_blocked2d import FIELDS, run, small
 from test_gpu_blocked3d import alone, strip
@@ -106,3 +106,25 @@ def test_blocked_3d_keeps_the_marchs_cells(nx, ny, nz, direction):
     assert any(not np.isfinite(x).all() for x in ref)
     for x, y in zip(got, ref):
         assert np.array_equal(x, y, equal_nan=True)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('scheme', ['tm', '3d'])
+def test_dft_planes_hold_the_compact_phasors(scheme):
+    """dft() and read_dft() form the same complex values (a zero frequency has
+    a NaN imaginary part beside an infinite real one)."""
+    s, fg = small('tm', 'float32', 97, 98, 70) if scheme == 'tm' else strip(64, 48, 120, 60)
+    freqs = np.array(s.sparam_freqs, float)
+    freqs[0] = 0.0
+    s = dataclasses.replace(infinite(s), sparam_freqs=freqs)
+    print('case', scheme, s.shape, flush=True)
+    dev = Solver(s, fg).run()
+    N, planes = s.num_cpml, dev.dft()
+    w = (slice(None), slice(N, s.ny - N)) if scheme == 'tm' else (slice(None), slice(N, s.nx - N), slice(N, s.ny - N))
+    assert any(not np.isfinite(z[w]).all() for z in planes.values())
+    for (k, port), z in planes.items():
+        ref = dev.read_dft(port - 1, COMP_KEYS[scheme].index(k)).reshape(z[w].shape)
+        for x, y in ((z[w].real, ref.real), (z[w].imag, ref.imag)):
+            assert np.array_equal(x, y, equal_nan=True)
+            assert np.array_equal(np.signbit(x)[~np.isnan(x)], np.signbit(y)[~np.isnan(y)])
+    dev.close()
