@@ -126,22 +126,6 @@ def _window(s):
     return None, (N, s.ny - N)
 
 
-def expand_dft(s, comp_arrays):
-    """Compact window phasors -> the reference's full-plane arrays (zeros outside)."""
-    nf = len(s.sparam_freqs)
-    wx, wy = _window(s)
-    out = {}
-    for key, z in comp_arrays.items():
-        if s.scheme == '3d':
-            full = np.zeros((nf, s.nx, s.ny), dtype=np.complex128)
-            full[:, wx[0]:wx[1], wy[0]:wy[1]] = z.reshape(nf, wx[1] - wx[0], wy[1] - wy[0])
-        else:
-            full = np.zeros((nf, s.ny), dtype=np.complex128)
-            full[:, wy[0]:wy[1]] = z.reshape(nf, wy[1] - wy[0])
-        out[key] = full
-    return out
-
-
 COMP_KEYS = {'tm': ('e', 'h'), 'te': ('e', 'h'), '3d': ('ex', 'ey', 'hx', 'hy')}
 FIELDS = {'tm': ('ez', 'hx', 'hy'), 'te': ('ex', 'ey', 'hz'), '3d': ('ex', 'ey', 'ez', 'hx', 'hy', 'hz')}
 
