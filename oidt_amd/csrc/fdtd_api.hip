@@ -1169,8 +1169,9 @@ int read_rows(oidt_batch* b, const char* src, size_t pitch, size_t row_len, size
 // put(piece, first byte, bytes) moves each piece to its place while the next
 // one is on its way.  (A copy straight into the caller's pageable array runs at
 // a few GB/s.)
+// `complex`: re, im pairs, given as re + 1j * im (k_pack_complex).
 template <typename Put>
-int read_pieces(oidt_batch* b, hipStream_t st, const void* src, size_t bytes, Put&& put) {
+int read_pieces(oidt_batch* b, hipStream_t st, const void* src, size_t bytes, Put&& put, bool complex = false) {
   struct Piece { int id; void* p; size_t at, n; };
   Piece prev{-1, nullptr, 0, 0};
   auto drain = [&](const Piece& pc) -> int {
@@ -1184,7 +1185,14 @@ int read_pieces(oidt_batch* b, hipStream_t st, const void* src, size_t bytes, Pu
     Piece pc{-1, nullptr, at, std::min(kReadPiece, bytes - at)};
     pc.id = b->staging.get(pc.n, &pc.p, prev.id);
     if (pc.id < 0) return fail(OIDT_ENOMEM, "pinned staging allocation failed");
-    HIP_TRY(hipMemcpyAsync(pc.p, static_cast<const char*>(src) + at, pc.n, hipMemcpyDeviceToHost, st));
+    if (complex) {
+      const unsigned n = (unsigned)(pc.n / sizeof(double2));
+      hipLaunchKernelGGL(k_pack_complex, dim3((n + kThreads - 1) / kThreads), dim3(kThreads), 0, st,
+                         reinterpret_cast<const double2*>(static_cast<const char*>(src) + at), n, static_cast<double2*>(pc.p));
+      HIP_TRY(hipGetLastError());
+    } else {
+      HIP_TRY(hipMemcpyAsync(pc.p, static_cast<const char*>(src) + at, pc.n, hipMemcpyDeviceToHost, st));
+    }
     if (b->staging.submit(pc.id, st) != 0) return fail(OIDT_EHIP, "event record failed");
     if (prev.id >= 0) rc = drain(prev);
     prev = pc;
@@ -1484,7 +1492,7 @@ namespace {
 // others: they are read on a stream of their own then, without waiting for
 // the batch stream.
 template <typename Put>
-int read_acc(oidt_batch* b, const SlotHost& sh, int32_t port, int32_t comp, Put&& put) {
+int read_acc(oidt_batch* b, const SlotHost& sh, int32_t port, int32_t comp, Put&& put, bool complex = false) {
   const oidt_run_desc& d = sh.desc;
   const size_t bytes = (size_t)d.nf * sh.wcells * 2 * sizeof(double);
   const size_t off = d.precision == OIDT_F64 ? layout<double>(d).off_acc : layout<float>(d).off_acc;
@@ -1494,7 +1502,7 @@ int read_acc(oidt_batch* b, const SlotHost& sh, int32_t port, int32_t comp, Put&
     st = b->aux;
   }
   return read_pieces(b, st, static_cast<char*>(sh.dmem) + off + (size_t)(port * (sh.nq / 2) + comp) * bytes, bytes,
-                     std::forward<Put>(put));
+                     std::forward<Put>(put), complex);
 }
 }  // namespace
 
@@ -1532,17 +1540,11 @@ int oidt_batch_read_dft_plane(oidt_batch* b, int32_t slot, int32_t port, int32_t
     for (size_t e = at / 16, end = (at + n) / 16; e < end;) {
       const size_t row = e / len, c = e - row * len, m = std::min(len - c, end - e);
       const size_t f = row / rows, x = x0 + row % rows;
-      // re + 1j * im as complex arithmetic forms it (a zero's sign, non-finite parts)
-      double* o = out + 2 * ((f * xs + x) * d.ny + N + c);
-      const double* v = reinterpret_cast<const double*>(p);
-      for (size_t k = 0; k < m; ++k) {
-        o[2 * k] = v[2 * k] + 0.0 * v[2 * k + 1];
-        o[2 * k + 1] = 0.0 + v[2 * k + 1];
-      }
+      std::memcpy(out + 2 * ((f * xs + x) * d.ny + N + c), p, m * 16);
       p += m * 16;
       e += m;
     }
-  });
+  }, true);
 }
 
 int oidt_batch_port_power(oidt_batch* b, int32_t slot, int32_t port, int32_t sub_slot, int32_t sub_port,
