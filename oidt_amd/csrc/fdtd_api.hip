@@ -2,9 +2,10 @@
 //
 // A batch owns a HIP stream (default priority), a device table of run
 // descriptors (Slot<T>), a tile list for the stencil kernels and a work list
-// for the DFT kernel.  One chunk = kChunk x (E launch, H launch) + DFT launch +
-// advance launch, captured once per batch composition as a hipGraph and
-// replayed.  A single run (oidt_solver) is a batch with one slot.
+// for the DFT kernel.  One chunk = the stencil launches of kChunk steps (two per
+// step, one in the fused form, one per 2..8 steps in the blocked forms) + DFT
+// launch + advance launch, captured once per batch composition as a hipGraph
+// and replayed.  A single run (oidt_solver) is a batch with one slot.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -888,6 +889,9 @@ void launch_fused(oidt_batch* b, int gs, int tstep) {
 // (TMz FP64); 1237 x 301 2.72 / 2.01 and 3.32 / 2.83; 64 guides of 800..4000 x
 // 240 155 / 57 (TMz FP32) and 158 / 59 (TEz FP32; 12 x 4: 69).  8 x 4 (the
 // depths 2 and 4 in FP32) takes 65 and 82 there, 8 x 8 tiles of 64 planes 67.
+// (With zero factors in place of the range selects, see blocked_step_2d; these
+// cost the narrow shapes 0..2 %, the wide ones 2..4 %: 64 other guides 140 / 50.6
+// before, 141 / 51.5 now.)
 template <typename T, int SCH, int TB>
 void launch_blocked2d(oidt_batch* b, int gs, int tstep) {
   const Slot<T>* sl = static_cast<const Slot<T>*>(b->d_slots);
@@ -912,8 +916,10 @@ void launch_blocked2d(oidt_batch* b, int gs, int tstep) {
       using all = integral_constant<int, SCH == SCHEME_TEZ ? (MON_A | MON_B) : (MON_A | MON_B | MON_C)>;
       if (b->tb_mon) {
         // with monitors: 16 x 2 while every tile has a CU of its own, else 8 x
-        // 4 (4170 x 430 TEz, two planes: 15.7 / 11.5 us per step; 287 x 235
-        // lossy TMz, three: 2.9 / 3.5; 48-plane tiles 12.5 and 4.1)
+        // 4 (us per step: 4170 x 430 TEz, two planes, 14.5 / 10.0; 152 x 195
+        // 2.2 / 2.5; lossy TMz, three planes, 2787 x 430 13.7 / 10.9; 132 x 195
+        // 2.7 / 3.5; 48-plane tiles, tried at 11.5 and 3.5 us for the 8 x 4
+        // shape, 12.5 and 4.1)
         if constexpr (sizeof(T) == 4)
           if (!b->tb_few) return go(i8{}, i4{}, i4{}, all{});
         return go(i16{}, i2{}, i4{}, all{});

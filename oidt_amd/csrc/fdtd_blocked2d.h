@@ -1,5 +1,5 @@
-// Temporally blocked 2D Yee step for gfx950 (TMz and TEz): TB time steps per
-// launch on register-resident tiles.
+// Temporally blocked 2D Yee step for gfx950 (TMz, TEz and the studies' lossy
+// TMz): TB time steps per launch on register-resident tiles.
 //
 // A block of W waves holds an extended tile of W*K planes (x) by 64 rows (y,
 // one per lane): wave w owns K planes, every lane its row of those planes.
@@ -28,7 +28,7 @@
 //
 // The arithmetic is written with explicit fused multiply-adds, the ones the
 // two-kernel forms (k_*_e2 / k_*_h2, k_tmzl_e / k_tmzl_h) compile to, so every
-// shape and every class gives the same bits.
+// shape and every class gives the same bits, infinite and NaN ones included.
 //
 // Field monitors.  The running DFTs of the study drivers (one per field, over
 // any box) ride along: their sums of the wave's cells sit in registers over
@@ -36,8 +36,9 @@
 // double, rounded to T), so a whole-plane phasor costs one read and one write
 // of its sums per 8 steps instead of a kernel per step.  us per step, two
 // kernels and the monitor kernel / blocked: TEz study 4170 x 430 with two
-// planes 36.8 / 11.5, lossy TMz 2787 x 430 with three 33.2 / 11.4, bound by the
-// conversions and FP64 operations of the fold.
+// planes 36.8 / 10.0 (11.2 with a branch per cell round the sums' loads), lossy
+// TMz 2787 x 430 with three 33.2 / 10.9, bound by the conversions and FP64
+// operations of the fold.
 #pragma once
 #include "fdtd_kernels.h"
 

@@ -2549,10 +2549,12 @@ __global__ __launch_bounds__(kThreads, 4) void k_3d_halo(const Slot<T>* __restri
 // and writes the inner cells' state after its steps to the other set.
 //
 // What bounds it: instruction issue and its three barriers per plane (one
-// 16-wave block per CU: 4.5 us per plane and two steps, near enough the same
-// where every tile has a CU of its own).  Rows inside every update range, in
-// tiles without z slab, source or capture, take a body without selects inside
-// the x limits, with the x and y psi terms behind uniform branches.  Each
+// 16-wave block per CU: 3.5 us per plane and two steps on large runs, 4.3..5.5
+// on small ones, whose slabs and limits take the general body more often; 45 %
+// of the vector rate and 51 % of the wave cycles in waits on the 16 guides).
+// Rows inside every update range, in tiles without z slab, source or capture,
+// take a body without selects inside the x limits, with the x and y psi terms
+// behind uniform branches.  Each
 // position waits once, at its start, for what the position before requested,
 // then stores the final plane and requests the next: the vector-memory counter
 // is in order, so a wait further down would also be for this position's own
@@ -2624,7 +2626,6 @@ __global__ __launch_bounds__(64 * W) void k_3d_tb(const Slot<T>* __restrict__ sl
     const int j = j0 - TB + w, k = k0 - TB + lane;
     const int jc = min(max(j, 0), ny - 1), kc = min(max(k, 0), nz - 1);
     const bool own = j >= j0 && j < j0 + TY && j < ny && k >= k0 && k < k0 + TZ && k < nz;
-    const bool jgrid = j >= 0 && j < ny;
     const int xo1 = min(x0 + kTb3Seg, nx);                       // inner planes [x0, xo1)
     const int xf = max(x0 - TB, 0), xl = min(xo1 - 1 + TB, nx - 1);   // loaded planes [xf, xl]
     const unsigned pl = (unsigned)ny * nz;
